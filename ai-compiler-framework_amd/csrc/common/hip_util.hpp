@@ -62,36 +62,22 @@ __device__ __forceinline__ uint32_t f32x2_to_bf16x2(float lo, float hi) {
 __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
   return static_cast<uint16_t>(f32x2_to_bf16x2(f, 0.0f));
 }
-// binary16 <-> fp32 with integer operations only.  The reference converts
-// with __half2float (exact) and __float2half_rn (one RNE rounding of the
-// fp32 value); doing the same here keeps hipcc from fusing a convert-fma-
-// convert chain into v_fma_mix*, which rounds the exact result straight to
-// f16 and can differ from the reference in the last bit.
+// binary16 <-> fp32 with the conversion instructions.  The reference converts
+// with __half2float (exact) and __float2half_rn (one RNE rounding of the fp32
+// value).  The empty asm keeps hipcc from fusing an fma and the conversion of
+// its result into v_fma_mixlo/mixhi_f16, which rounds the exact result straight
+// to f16 and can differ from the reference in the last bit.  (A conversion of
+// an operand may be fused: it is exact.)  Every NaN becomes the quiet NaN
+// without payload, with its sign.  Bits of the integer formulation used
+// before, which took ~12 VALU instructions and two branches a value; here 4.
 __device__ __forceinline__ float f16_to_f32(uint16_t h) {
-  const uint32_t sign = (uint32_t)(h & 0x8000u) << 16;
-  const uint32_t e = (h >> 10) & 0x1fu, m = h & 0x3ffu;
-  if (e == 0) {
-    // zero / subnormal: m * 2^-24 is exact in fp32
-    const float v = (float)m * 5.9604644775390625e-8f;
-    return __uint_as_float(__float_as_uint(v) | sign);
-  }
-  if (e == 31) return __uint_as_float(sign | 0x7f800000u | (m << 13));
-  return __uint_as_float(sign | ((e + 112u) << 23) | (m << 13));
+  return static_cast<float>(__builtin_bit_cast(_Float16, h));
 }
 __device__ __forceinline__ uint16_t f32_to_f16(float f) {
-  uint32_t x = __float_as_uint(f);
-  const uint16_t sign = (uint16_t)((x >> 16) & 0x8000u);
-  x &= 0x7fffffffu;
-  if (x >= 0x7f800000u) return sign | (x > 0x7f800000u ? 0x7e00u : 0x7c00u);  // NaN / inf
-  if (x >= 0x477ff000u) return sign | 0x7c00u;  // >= 65520 rounds to inf
-  if (x >= 0x38800000u) {                       // normal binary16 range
-    x += 0xc8000fffu + ((x >> 13) & 1u);        // rebias exponent, round half to even
-    return sign | (uint16_t)(x >> 13);
-  }
-  // subnormal / zero: adding 0.5 aligns the 2^-24 quantum to the fp32 ulp,
-  // so the fp32 addition performs the RNE rounding
-  const float r = __uint_as_float(x) + 0.5f;
-  return sign | (uint16_t)(__float_as_uint(r) - 0x3f000000u);
+  const uint32_t u = __float_as_uint(f);
+  float q = __uint_as_float(f == f ? u : ((u | 0x7fffffffu) & 0xffc00000u));
+  asm("" : "+v"(q));
+  return __builtin_bit_cast(uint16_t, static_cast<_Float16>(q));
 }
 
 // ---- wave64 reductions (butterfly over all 64 lanes) ----------------------
