@@ -123,7 +123,15 @@ __device__ __forceinline__ float gelu_tanh_grad_f(float x) {
 __device__ __forceinline__ void block_mean_f64(const float* __restrict__ v, int64_t n,
                                                float* __restrict__ out, double* red) {
   double acc = 0.0;
-  for (int64_t i = threadIdx.x; i < n; i += 256) acc += (double)v[i];
+  int64_t i = threadIdx.x;
+  for (; i + 15 * 256 < n; i += 16 * 256) {  // 16 loads in flight, added in order
+    float q[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) q[u] = v[i + u * 256];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) acc += (double)q[u];
+  }
+  for (; i < n; i += 256) acc += (double)v[i];
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;

@@ -10,8 +10,9 @@
 // Row kernels keep a whole row in registers: a row is owned by LPR lanes
 // (a fraction of a wave, one wave, or several waves of one workgroup), each
 // holding VPT 16-byte vectors, so X is read from HBM exactly once and every
-// output is written once.  Shapes that do not match a register-resident
-// configuration use a looping kernel that reads the row twice.
+// output is written once.  Rows of any length from 4 to 32768 columns at any
+// 4-byte alignment; shorter and longer rows use a looping kernel that reads
+// the row two or three times.
 #include "../common/hip_util.hpp"
 
 namespace aicf::hip {
@@ -449,7 +450,17 @@ __device__ __forceinline__ RowStat stat_shfl(const RowStat& v, int off) {
 // then scale each lane's exponentials by exp(m_lane - M) / S.  A row whose
 // values are all equal gets exactly 1/C when C is a power of two (every
 // exponential and scale factor is then exactly 1 and S = C).
-template <int LPR, int VPT, int MODE>
+//
+// RAG: any C >= 4 up to LPR VPT 4, any 4-byte alignment (the loads and stores
+// are 16 bytes at element addresses, which gfx950 takes unaligned).  The
+// vectors past the last whole one are moved back to end at column C - 1, so
+// every load lies in the row, and their elements that an earlier vector holds
+// become -inf: they add nothing to a maximum or to a sum of exponentials, are
+// left out of the plain sums, and are not stored.  [4096, 10007] cross-entropy:
+// 122 us on the looping kernel (three 4-byte reads), 58 here (5.7 TB/s; bound
+// by HBM).
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+template <int LPR, int VPT, int MODE, bool RAG>
 __global__ __launch_bounds__(LPR >= 256 ? LPR : 256) void row_reg_kernel(RowArgs a) {
   constexpr int THREADS = LPR >= 256 ? LPR : 256;
   constexpr int RPB = THREADS / LPR;            // rows per workgroup
@@ -466,24 +477,49 @@ __global__ __launch_bounds__(LPR >= 256 ? LPR : 256) void row_reg_kernel(RowArgs
   const f32x4* xr = reinterpret_cast<const f32x4*>(a.x + (active ? row : 0) * C);
   // cross-entropy: the label is read first, so its latency hides behind the row loads
   const int lab = (MODE == MODE_XENT && active) ? a.labels[row] : -1;
+  const int end = (int)C - 4;  // (RAG) first column of the last vector
+  auto col = [&](int k) { return RAG ? min((k * LPR + l) * 4, end) : (k * LPR + l) * 4; };
+  // (RAG) first element of vector k that no earlier vector holds; 4: none
+  auto first = [&](int k) { return RAG ? min(max((k * LPR + l) * 4 - end, 0), 4) : 0; };
 
   // an inactive row (past R, uniform across its lanes) reads row 0 and
   // stores nothing: the loads need no predicate
   f32x4 v[VPT];
 #pragma unroll
-  for (int k = 0; k < VPT; ++k) v[k] = __builtin_nontemporal_load(xr + k * LPR + l);
+  for (int k = 0; k < VPT; ++k) {
+    if constexpr (RAG)
+      v[k] = __builtin_nontemporal_load(reinterpret_cast<const f32x4u*>(reinterpret_cast<const float*>(xr) + col(k)));
+    else
+      v[k] = __builtin_nontemporal_load(xr + k * LPR + l);
+  }
+  if constexpr (RAG) {
+#pragma unroll
+    for (int k = 0; k < VPT; ++k)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (j < first(k)) v[k][j] = MODE == MODE_SUM ? 0.0f : -INFINITY;
+  }
 
   // this lane's statistics
   RowStat st{v[0][0], 0.0f, 0.0f, l * 4};
   if constexpr (MODE == MODE_SUM || MODE == MODE_SOFTMAX) {
 #pragma unroll
-    for (int k = 0; k < VPT; ++k) st.sx += (v[k][0] + v[k][1]) + (v[k][2] + v[k][3]);
+    for (int k = 0; k < VPT; ++k) {
+      if constexpr (RAG && MODE == MODE_SOFTMAX) {
+        const int f = first(k);
+        st.sx += ((f > 0 ? 0.0f : v[k][0]) + (f > 1 ? 0.0f : v[k][1])) +
+                 ((f > 2 ? 0.0f : v[k][2]) + (f > 3 ? 0.0f : v[k][3]));
+      } else {
+        st.sx += (v[k][0] + v[k][1]) + (v[k][2] + v[k][3]);
+      }
+    }
   }
   // cross-entropy: the label's logit sits in lane lab_l, vector lab_k,
-  // element lab & 3 (no lane for a label outside [0, C))
+  // element lab & 3 (RAG, the last vector: lab - end); no lane for a label
+  // outside [0, C)
   const int lab_q = lab >> 2;
-  const bool lab_here = MODE == MODE_XENT && lab >= 0 && lab_q % LPR == l;
-  const int lab_k = lab_q / LPR, lab_j = lab & 3;
+  const bool lab_here = MODE == MODE_XENT && lab >= 0 && (!RAG || lab < (int)C) && lab_q % LPR == l;
+  const int lab_k = lab_q / LPR, lab_j = RAG && lab_q * 4 > end ? lab - end : lab & 3;
   if constexpr (MODE == MODE_XENT) {
     // the lane's maximum, then the first column holding it (for finite
     // values the result of a running strict-greater scan), then the
@@ -495,7 +531,7 @@ __global__ __launch_bounds__(LPR >= 256 ? LPR : 256) void row_reg_kernel(RowArgs
 #pragma unroll
     for (int k = VPT - 1; k >= 0; --k)
 #pragma unroll
-      for (int j = 3; j >= 0; --j) idx = v[k][j] == m ? (k * LPR + l) * 4 + j : idx;
+      for (int j = 3; j >= 0; --j) idx = v[k][j] == m ? col(k) + j : idx;
     float zl = 0.0f;
 #pragma unroll
     for (int k = 0; k < VPT; ++k)
@@ -551,13 +587,25 @@ __global__ __launch_bounds__(LPR >= 256 ? LPR : 256) void row_reg_kernel(RowArgs
   }
   const float c = (m_lane == st.m ? 1.0f : __expf(m_lane - st.m)) / st.s;
   f32x4* yr = reinterpret_cast<f32x4*>(a.y + row * C);
+  [[maybe_unused]] auto put_rag = [&](int k, const f32x4& o) {
+    const int f = first(k);
+    float* p = a.y + row * C + col(k);
+    if (f == 0) {
+      __builtin_nontemporal_store(o, reinterpret_cast<f32x4u*>(p));
+    } else {  // one lane of the row at most has 0 < f < 4
+#pragma unroll
+      for (int j = 1; j < 4; ++j)
+        if (j >= f) p[j] = o[j];
+    }
+  };
   if constexpr (MODE == MODE_SOFTMAX) {
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
       f32x4 o;
 #pragma unroll
       for (int j = 0; j < 4; ++j) o[j] = v[k][j] * c;
-      __builtin_nontemporal_store(o, yr + k * LPR + l);
+      if constexpr (RAG) put_rag(k, o);
+      else __builtin_nontemporal_store(o, yr + k * LPR + l);
     }
     if (l == 0) {
       if (a.rmax) a.rmax[row] = st.m;
@@ -572,7 +620,8 @@ __global__ __launch_bounds__(LPR >= 256 ? LPR : 256) void row_reg_kernel(RowArgs
 #pragma unroll
       for (int j = 0; j < 4; ++j)  // (p - onehot) / B
         o[j] = (v[k][j] * c - ((lab_here && k == lab_k && j == lab_j) ? 1.0f : 0.0f)) * sc;
-      __builtin_nontemporal_store(o, yr + k * LPR + l);
+      if constexpr (RAG) put_rag(k, o);
+      else __builtin_nontemporal_store(o, yr + k * LPR + l);
     }
     if (l == 0) {
       a.argmax[row] = st.i;
@@ -661,8 +710,8 @@ __global__ __launch_bounds__(256) void mean_kernel(const float* __restrict__ v, 
   block_mean_f64(v, n, out, red);
 }
 
-// Picks a register-resident configuration when C is one of the row widths
-// it covers, else the looping kernel.
+// Picks a register-resident configuration: one of the exact row widths, or
+// the smallest that holds the row; the looping kernel for C < 4 and C > 32768.
 template <int MODE>
 Status launch_rows(const RowArgs& a, void* stream) {
   hipStream_t s = as_stream(stream);
@@ -673,7 +722,7 @@ Status launch_rows(const RowArgs& a, void* stream) {
     constexpr int RPB = (LPR) >= 256 ? 1 : 256 / (LPR);                                       \
     constexpr int THREADS = (LPR) >= 256 ? (LPR) : 256;                                       \
     static_assert(THREADS <= 1024, "row too wide");                                          \
-    row_reg_kernel<LPR, VPT, MODE><<<(unsigned)((R + RPB - 1) / RPB), THREADS, 0, s>>>(a);  \
+    row_reg_kernel<LPR, VPT, MODE, false><<<(unsigned)((R + RPB - 1) / RPB), THREADS, 0, s>>>(a);  \
     return launch_status("row_kernel");                                                      \
   }
   if constexpr (MODE == MODE_SOFTMAX) {
@@ -701,6 +750,34 @@ Status launch_rows(const RowArgs& a, void* stream) {
   ROW_CASE(512, 8)    // C = 16384
   ROW_CASE(512, 16)   // C = 32768
 #undef ROW_CASE
+  // any other width or alignment: the fewest lanes that hold the row
+#define ROW_RAG(LPR, VPT)                                                                         \
+  if (C <= (int64_t)(LPR) * (VPT) * 4) {                                                          \
+    constexpr int RPB = (LPR) >= 256 ? 1 : 256 / (LPR);                                           \
+    constexpr int THREADS = (LPR) >= 256 ? (LPR) : 256;                                           \
+    row_reg_kernel<LPR, VPT, MODE, true><<<(unsigned)((R + RPB - 1) / RPB), THREADS, 0, s>>>(a);  \
+    return launch_status("row_kernel");                                                           \
+  }
+  if (C >= 4) {
+    ROW_RAG(16, 1)
+    ROW_RAG(16, 2)
+    ROW_RAG(32, 2)
+    ROW_RAG(64, 2)
+    ROW_RAG(128, 2)
+    ROW_RAG(128, 3)
+    ROW_RAG(128, 4)
+    ROW_RAG(256, 3)
+    ROW_RAG(256, 4)
+    ROW_RAG(256, 6)
+    ROW_RAG(256, 8)
+    ROW_RAG(512, 5)
+    ROW_RAG(512, 6)
+    ROW_RAG(512, 8)
+    ROW_RAG(512, 10)
+    ROW_RAG(512, 12)
+    ROW_RAG(512, 16)
+  }
+#undef ROW_RAG
   row_loop_kernel<MODE><<<(unsigned)R, 256, 0, s>>>(a);
   return launch_status("row_loop_kernel");
 }
