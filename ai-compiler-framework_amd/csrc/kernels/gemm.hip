@@ -31,101 +31,12 @@
 #include <type_traits>
 #include <utility>
 
-#include "../common/adamw.hpp"
-#include "../common/hip_util.hpp"
+#include "../common/gemm_types.hpp"
 #include "../common/smallstep.hpp"
 
 namespace aicf::hip {
 
 namespace {
-
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-
-enum InKind { IN_F32 = 0, IN_F16 = 1, IN_BF16 = 2 };
-enum OutKind { OUT_F32 = 0, OUT_F16 = 1, OUT_BF16 = 2 };
-// ACT_ADAMW (fp32 accumulators only): the tile is the gradient of a weight
-// matrix; the epilogue applies AdamW to that weight instead of storing it.
-enum Act { ACT_NONE = 0, ACT_RELU = 1, ACT_GELU = 2, ACT_DGELU = 3, ACT_ADAMW = 4 };
-
-// Optimizer state a fused weight-gradient GEMM updates in place ([M, N]
-// row-major like the output, leading dimension ldc).
-struct GemmAdamW {
-  float* P;             // fp32 master weights
-  float* M;             // first moment
-  float* V;             // second moment
-  uint16_t* Wb;         // bf16 shadow of P
-  const int32_t* step;  // device step counter (already incremented)
-  AdamWArgs args;
-};
-enum LoadMode { LD_KCONTIG = 0, LD_MNCONTIG = 1, LD_GATHER = 2 };
-
-struct GemmParams {
-  const void* A;
-  const void* B;
-  void* C;
-  const void* bias;  // nullptr = no bias
-  void* aux;         // pre-activation out (GELU) or Z in (DGELU); nullptr = none
-  int64_t M, N, K;
-  int64_t a_rs, a_cs;  // logical A[M,K] strides (elements)
-  int64_t b_rs, b_cs;  // logical B[K,N] strides
-  int64_t c_rs, c_cs;
-  int64_t bias_s;
-  int64_t aux_rs;
-  int a_mode, b_mode;
-  int act;
-  int bias_f32;  // bias stored as fp32 (else in the output type)
-  int tiles_m, tiles_n;
-  GemmAdamW adam;  // ACT_ADAMW only
-  float* colsum;   // ACT_DGELU, bf16 out: per-tile column sums of C, row m0/256 of [M/256, N]
-};
-
-template <int IN>
-struct InTraits;
-template <>
-struct InTraits<IN_F32> {
-  typedef float T;
-  static constexpr int CE = 4;    // elements per 16-byte chunk
-  static constexpr int KPM = 2;   // K per MFMA
-  static constexpr int EPL = 1;   // elements per lane per MFMA operand
-};
-template <>
-struct InTraits<IN_F16> {
-  typedef uint16_t T;
-  static constexpr int CE = 8;
-  static constexpr int KPM = 16;
-  static constexpr int EPL = 8;
-};
-template <>
-struct InTraits<IN_BF16> {
-  typedef uint16_t T;
-  static constexpr int CE = 8;
-  static constexpr int KPM = 16;
-  static constexpr int EPL = 8;
-};
-
-template <int OUT>
-__device__ __forceinline__ void store_out(void* base, int64_t idx, float v) {
-  if constexpr (OUT == OUT_F32) {
-    ((float*)base)[idx] = v;
-  } else if constexpr (OUT == OUT_F16) {
-    ((uint16_t*)base)[idx] = f32_to_f16(v);
-  } else {
-    ((uint16_t*)base)[idx] = f32_to_bf16(v);
-  }
-}
-template <int OUT>
-__device__ __forceinline__ float load_out(const void* base, int64_t idx) {
-  if constexpr (OUT == OUT_F32) {
-    return ((const float*)base)[idx];
-  } else if constexpr (OUT == OUT_F16) {
-    return f16_to_f32(((const uint16_t*)base)[idx]);
-  } else {
-    return bf16_to_f32(((const uint16_t*)base)[idx]);
-  }
-}
 
 // XOR swizzle of the 16-byte chunk index inside one LDS row.
 template <int NCH>
@@ -212,67 +123,6 @@ struct TileLoader {
   }
 };
 
-template <int IN>
-__device__ __forceinline__ floatx16 mfma32(const typename InTraits<IN>::T* a,
-                                          const typename InTraits<IN>::T* b, floatx16 acc);
-
-template <>
-__device__ __forceinline__ floatx16 mfma32<IN_F32>(const float* a, const float* b, floatx16 acc) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(a[0], b[0], acc, 0, 0, 0);
-}
-template <>
-__device__ __forceinline__ floatx16 mfma32<IN_BF16>(const uint16_t* a, const uint16_t* b,
-                                                   floatx16 acc) {
-  const bf16x8 av = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u16x8*>(a));
-  const bf16x8 bv = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u16x8*>(b));
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc, 0, 0, 0);
-}
-template <>
-__device__ __forceinline__ floatx16 mfma32<IN_F16>(const uint16_t* a, const uint16_t* b,
-                                                  floatx16 acc) {
-  const f16x8 av = __builtin_bit_cast(f16x8, *reinterpret_cast<const u16x8*>(a));
-  const f16x8 bv = __builtin_bit_cast(f16x8, *reinterpret_cast<const u16x8*>(b));
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bv, acc, 0, 0, 0);
-}
-
-// 16 x 16 x 32 MFMA (16-bit operands): a lane holds 8 consecutive K of one
-// row of each operand; the 16 x 16 fp32 result has row (lane & 15) of the
-// A operand and 4 consecutive columns 4 (lane >> 4) .. +3 of the B operand.
-// Same flops per issue cycle as 32 x 32 x 16 with a quarter of the
-// accumulator registers per instruction: it moves half the accumulator bits
-// per flop, and on this power-limited part it sustains a ~10% higher clock.
-template <int IN>
-__device__ __forceinline__ floatx4 mfma16(const uint16_t* a, const uint16_t* b, floatx4 acc) {
-  if constexpr (IN == IN_BF16) {
-    const bf16x8 av = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u16x8*>(a));
-    const bf16x8 bv = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u16x8*>(b));
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc, 0, 0, 0);
-  } else {
-    const f16x8 av = __builtin_bit_cast(f16x8, *reinterpret_cast<const u16x8*>(a));
-    const f16x8 bv = __builtin_bit_cast(f16x8, *reinterpret_cast<const u16x8*>(b));
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bv, acc, 0, 0, 0);
-  }
-}
-
-// Grouped raster: workgroup w of XCD x (dispatch order w*8+x) gets
-// tile (tm, tn) so that each XCD sweeps a contiguous run of tiles and
-// GROUP_M consecutive tile rows share B columns in its L2.
-__device__ __forceinline__ void tile_coords_of(int id, int tiles_m, int tiles_n, int& tm, int& tn) {
-  const int total = tiles_m * tiles_n;
-  // XCD-aware remap: hardware id i runs on XCD (i % 8); give every XCD a
-  // contiguous range of logical ids.
-  if ((total & 7) == 0) {
-    const int per = total >> 3;
-    id = (id & 7) * per + (id >> 3);
-  }
-  constexpr int GROUP_M = 4;  // measured best on MI355X for 256x256 tiles
-  const int group = id / (GROUP_M * tiles_n);
-  const int first_m = group * GROUP_M;
-  const int gsize = (tiles_m - first_m) < GROUP_M ? (tiles_m - first_m) : GROUP_M;
-  const int in_group = id % (GROUP_M * tiles_n);
-  tm = first_m + in_group % gsize;
-  tn = in_group / gsize;
-}
 __device__ __forceinline__ void tile_coords(int tiles_m, int tiles_n, int& tm, int& tn) {
   tile_coords_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
 }
@@ -923,13 +773,6 @@ struct NTSched {
 // them take the four 32-byte slots: chunk pair XOR (bit 1, bit 3) of k.
 // Every form keeps rows k and k + 4 (k % 8 < 4) alike, as the fragment's
 // second read (4 rows on) reuses the first one's column.
-template <int MS, int ES = 2, int CPR = 16>
-__device__ __forceinline__ int nt_mn_swizzle(int k) {
-  if constexpr (ES == 4) return 8 * ((k >> 2) & 1);
-  if constexpr (CPR == 8) return 2 * (((k >> 1) & 1) | (((k >> 3) & 1) << 1));
-  return MS == 16 ? ((4 * (k & 3)) ^ (2 * ((k >> 3) & 1))) : 4 * (k & 3);
-}
-
 template <bool KC, int BMN, int NW, int ES>
 struct NTOperand {
   static constexpr int BYTES = BMN * 128;            // a stage holds 128 B of K per row
@@ -1573,9 +1416,14 @@ Status run_gemm(GemmParams& p, hipStream_t s) {
   if constexpr (IN == IN_F32 && OUT == OUT_F32) {
     // fewer than 128 tiles of 64 x 64: one 16 x 16 tile per wave with K split
     // over the waves of a workgroup reaches more CUs than any tiled
-    // configuration, and reads every operand layout in place
+    // configuration, and reads every operand layout in place.  Above 512
+    // such tiles (two workgroups a CU) it re-reads the operands from L2 too
+    // often: 512^3 11.2 us against 7.1 on the edge kernel's K-split tiles,
+    // 300 x 1001 x 2000 50 against 30, but 300 x 300 x 1000 9.3 against 11.0.
     const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64);
-    if (tiles64 < kSmallGemmMaxTiles64 && (p.act == ACT_NONE || p.act == ACT_RELU) && p.c_cs == 1 && !p.aux) {
+    const int64_t tiles16 = ((p.M + 15) / 16) * ((p.N + 15) / 16);
+    const bool split = tiles16 > 512 && p.K >= 256 && edge_gemm_ok(p, IN);
+    if (tiles64 < kSmallGemmMaxTiles64 && !split && (p.act == ACT_NONE || p.act == ACT_RELU) && p.c_cs == 1 && !p.aux) {
       SmallGemm g{};
       g.A = (const float*)p.A;
       g.B = (const float*)p.B;
@@ -1639,6 +1487,14 @@ Status run_gemm(GemmParams& p, hipStream_t s) {
       }
       return run_nt<IN, OUT, 128, 128, 2, 2, true>(p, s);
     }
+    // at most one 32 x 32 tile a CU and K >= 2048: the edge kernel splits K
+    // eight ways (64 x 256 x 4096 11.6 -> 9.7 us, 256 x 1024 x 4096 12.0 ->
+    // 10.5 against the 64 x 64 tiles with 8 stages)
+    if constexpr (IN != IN_F32) {
+      const int64_t tiles32 = ((p.M + 31) / 32) * ((p.N + 31) / 32);
+      if (tiles32 <= 256 && p.K >= 2048 && p.a_mode == LD_KCONTIG && edge_gemm_ok(p, IN))
+        return edge_gemm(p, IN, OUT, s);
+    }
     // fewer tiles than CUs at 128x128: 64x64 tiles (4 waves of 32x32)
     if (nt_eligible<IN, OUT>(p, 64, 64, MN64)) {
       if constexpr (IN != IN_F32) {
@@ -1653,8 +1509,12 @@ Status run_gemm(GemmParams& p, hipStream_t s) {
       return run_nt<IN, OUT, 128, 128, 2, 2, true>(p, s);
     }
   }
-  // Large problems: 128x128 workgroup tiles (4 waves, 64x64 per wave).
-  // Smaller ones: 64x64 tiles so that enough workgroups exist.
+  // shapes no tile divides, unaligned rows
+  if (edge_gemm_ok(p, IN)) return edge_gemm(p, IN, OUT, s);
+  // What is left: strides with no contiguous dimension, a strided output, K
+  // or a contiguous extent of less than 16 bytes.  Large problems: 128x128
+  // workgroup tiles (4 waves, 64x64 per wave).  Smaller ones: 64x64 tiles so
+  // that enough workgroups exist.
   const int64_t big_tiles = ((p.M + 127) / 128) * ((p.N + 127) / 128);
   if (big_tiles >= 512) return run_cfg<IN, OUT, 128, 128, (IN == IN_F32 ? 32 : 64), 2, 2>(p, s);
   return run_cfg<IN, OUT, 64, 64, (IN == IN_F32 ? 32 : 64), 2, 2>(p, s);
