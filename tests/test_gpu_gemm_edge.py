@@ -2,7 +2,8 @@
 ends inside a 16-byte chunk, a chunk and a K-step early or late, edge tiles of
 one row or column, odd leading dimensions and odd base addresses, in all four
 operand layouts and every epilogue; each of the kernel's tile and K-split
-configurations.  Operands and outputs are views into memory full of NaN: a
+configurations; and shapes whose last exact tiles overlap their neighbours.
+Operands and outputs are views into memory full of NaN: a
 load that reads past an edge and counts, or a store outside the output, shows.
 
 Tolerances (normwise against fp64 products of the stored operands): fp32
@@ -61,7 +62,10 @@ SIZES = [(1, 1, 8, 0, 0), (9, 3, 8, 1, 1), (64, 64, 9, 0, 0), (17, 10, 15, 3, 2)
          (1030, 1029, 72, 0, 0), (2049, 520, 40, 1, 1),  # 64 x 64 tiles, short K
          (2050, 1031, 265, 1, 1), (1100, 2051, 784, 0, 0),  # 128 x 64
          (2561, 2051, 255, 0, 0), (2600, 2500, 264, 8, 8),  # 128 x 128
-         (3600, 3599, 520, 0, 0), (3333, 4099, 1000, 0, 1)]  # 256 x 256
+         (3600, 3599, 520, 0, 0), (3333, 4099, 1000, 0, 1),  # 256 x 256
+         # whole K-steps: the exact tiles, the last ones moved back (64, 128 and 256 wide, each pipeline depth)
+         (250, 248, 128, 0, 0), (249, 248, 1024, 8, 8), (1530, 1400, 192, 0, 0), (1528, 1400, 1024, 0, 0),
+         (2810, 3064, 128, 0, 0), (2808, 3064, 576, 8, 8), (4090, 4088, 128, 0, 0)]
 
 
 @pytest.mark.parametrize("dt", ["f32", "f16", "bf16", "bf16_f32"])
