@@ -187,48 +187,58 @@ __global__ __launch_bounds__(256) void colsum_finish_kernel(const float* __restr
 // 128-byte lines, are given to workgroups on one XCD (workgroup i runs on
 // XCD i % 8), so each line is fetched into one L2.  [8192, 4096] bf16: 16.6
 // us (4 lanes, 8 loads, no remap: 25.6 us; 1 lane: 23.3 us).
+//
+// THREADS 1024 (512 row slots) where there are few column blocks; RAG: any N
+// of at least a vector, any alignment: the last vector is moved back to end at
+// column N - 1 (columns that two lanes hold get the same bits from both).
 constexpr int kNarrowLanes = 2;
-constexpr int kNarrowSlots = 256 / kNarrowLanes;
 
-template <typename TI, bool BF16IN, bool OUT_F16>
-__global__ __launch_bounds__(256) void colsum_narrow_kernel(const TI* __restrict__ x, void* __restrict__ out,
-                                                            int64_t M, int64_t N) {
+template <typename TI, bool BF16IN, bool OUT_F16, int THREADS, bool RAG>
+__global__ __launch_bounds__(THREADS) void colsum_narrow_kernel(const TI* __restrict__ x, void* __restrict__ out,
+                                                                int64_t M, int64_t N) {
   constexpr int VEC = 16 / sizeof(TI);
   constexpr int CB = kNarrowLanes * VEC;  // columns per workgroup
+  constexpr int SLOTS = THREADS / kNarrowLanes;
   constexpr int UNROLL = 4;
-  __shared__ float red[kNarrowSlots][CB + 1];
+  typedef TI rvec __attribute__((ext_vector_type(VEC), aligned(sizeof(TI))));
+  __shared__ float red[SLOTS][CB + 1];
   const int slot = (int)threadIdx.x / kNarrowLanes, v = (int)threadIdx.x % kNarrowLanes;
   int bid = blockIdx.x;  // column block: XCD-contiguous when the grid is a multiple of 8
   if ((gridDim.x & 7) == 0) bid = (bid & 7) * (gridDim.x >> 3) + (bid >> 3);
   const int64_t c0 = (int64_t)bid * CB + v * VEC;
+  const int64_t at = RAG && c0 > N - VEC ? N - VEC : c0;
+  auto get = [&](int64_t r) -> uint4 {
+    if constexpr (RAG) return __builtin_bit_cast(uint4, *reinterpret_cast<const rvec*>(x + r * N + at));
+    else return *reinterpret_cast<const uint4*>(x + r * N + c0);
+  };
   float acc[VEC];
 #pragma unroll
   for (int e = 0; e < VEC; ++e) acc[e] = 0.0f;
-  if (c0 < N) {  // N % VEC == 0: the whole vector is in range
+  if (c0 < N) {  // the whole vector is in range: N % VEC == 0, or moved back
     int64_t r = slot;
-    for (; r + (UNROLL - 1) * kNarrowSlots < M; r += UNROLL * kNarrowSlots) {
+    for (; r + (UNROLL - 1) * SLOTS < M; r += UNROLL * SLOTS) {
       uint4 q[UNROLL];
 #pragma unroll
-      for (int u = 0; u < UNROLL; ++u)
-        q[u] = *reinterpret_cast<const uint4*>(x + (r + u * kNarrowSlots) * N + c0);
+      for (int u = 0; u < UNROLL; ++u) q[u] = get(r + u * SLOTS);
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) add_vec16<TI, BF16IN>(acc, q[u]);
     }
-    for (; r < M; r += kNarrowSlots) add_vec16<TI, BF16IN>(acc, *reinterpret_cast<const uint4*>(x + r * N + c0));
+    for (; r < M; r += SLOTS) add_vec16<TI, BF16IN>(acc, get(r));
   }
 #pragma unroll
   for (int e = 0; e < VEC; ++e) red[slot][v * VEC + e] = acc[e];
   __syncthreads();
-  for (int half = kNarrowSlots / 2; half > 0; half >>= 1) {  // slot i += slot i + half
-    for (int t = (int)threadIdx.x; t < half * CB; t += 256) {
+  for (int half = SLOTS / 2; half > 0; half >>= 1) {  // slot i += slot i + half
+    for (int t = (int)threadIdx.x; t < half * CB; t += THREADS) {
       const int i = t / CB, c = t % CB;
       red[i][c] += red[i + half][c];
     }
     __syncthreads();
   }
   if ((int)threadIdx.x < CB) {
-    const int64_t col = (int64_t)bid * CB + threadIdx.x;
-    if (col < N) {
+    const int64_t first = (int64_t)bid * CB + (threadIdx.x / VEC) * VEC;  // of this column's vector
+    const int64_t col = (RAG && first > N - VEC ? N - VEC : first) + threadIdx.x % VEC;
+    if (first < N) {
       const float sum = red[0][threadIdx.x];
       if constexpr (OUT_F16)
         ((uint16_t*)out)[col] = f32_to_f16(sum);
@@ -280,10 +290,22 @@ Status colsum_run(const void* x, void* out, float* partial, int64_t P, int64_t M
     partial = nullptr;
   }
   const int64_t gn = (N + kNarrowLanes * VEC - 1) / (kNarrowLanes * VEC);
-  if (vec && !partial && gn <= INT32_MAX) {
+  if (N >= VEC && !partial && gn <= INT32_MAX) {
     // one output, no partials: narrow column blocks over all rows (a
-    // [8192, 4096] bf16 sum on 8 workgroups of 512 columns took 133 us)
-    colsum_narrow_kernel<TI, BF16IN, OUT_F16><<<(unsigned)gn, 256, 0, s>>>((const TI*)x, out, M, N);
+    // [8192, 4096] bf16 sum on 8 workgroups of 512 columns took 133 us).
+    // At most 128 blocks (half the CUs): 1024 threads.  The f32 backward of
+    // 777 x 1000 x 523, whose [777, 523] sum took 9.8 us on scalar columns of
+    // 9 workgroups: 48.8 -> 39.1 us.
+    const TI* xp = (const TI*)x;
+#define NARROW(T, R) colsum_narrow_kernel<TI, BF16IN, OUT_F16, T, R><<<(unsigned)gn, T, 0, s>>>(xp, out, M, N)
+    if (gn <= 128 && M > 256) {
+      if (vec) NARROW(1024, false);
+      else NARROW(1024, true);
+    } else {
+      if (vec) NARROW(256, false);
+      else NARROW(256, true);
+    }
+#undef NARROW
     return launch_status(what);
   }
   if (vec)

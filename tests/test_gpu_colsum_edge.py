@@ -1,0 +1,33 @@
+"""GPU parity of the one-output column sum at widths that are no multiple of a
+16-byte vector, at odd base addresses, and around the switch to 1024 threads
+(M = 256, 128 column blocks), f32, f16 and bf16 in, against fp64: 1e-5 for
+fp32 outputs (sums of at most 4100 values), one rounding for f16 ones."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DT = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
+
+
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16", "f16_f16"])
+@pytest.mark.parametrize("M,N", [(1, 4), (3, 8), (5, 9), (777, 523), (256, 17), (257, 17), (4100, 10), (4099, 31),
+                                 (2048, 1024), (300, 1025), (300, 2049), (1000, 3), (513, 4099)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_column_sum_edges(C, M, N, dt, offset):
+    din = DT[dt.split("_")[0]]
+    dout = torch.float16 if "_" in dt else torch.float32
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + N)
+    full = torch.full((M * N + 64,), float("nan"), device="cuda", dtype=din)
+    x = full[16 + offset:16 + offset + M * N].view(M, N)
+    x.copy_(torch.randn((M, N), device="cuda", generator=g) + 0.25)
+    of = torch.full((N + 64,), 77.0, device="cuda", dtype=dout)
+    o = of[16:16 + N]
+    C.op_call(C.OpKind.ReduceSum, [x], [o])
+    ref = x.double().sum(0)
+    tol = 1e-5 if dout == torch.float32 else 2.0 ** -11 + 1e-5
+    assert float((o.double() - ref).abs().max() / ref.abs().max()) < tol
+    assert bool((of[:16] == 77).all()) and bool((of[16 + N:] == 77).all())
