@@ -243,7 +243,7 @@ __device__ __forceinline__ void row_sum2(float& a, float& b, f32x2_t* lds) {
   }
 }
 
-constexpr int ln_threads(int lpr) { return lpr > 256 ? lpr : 256; }
+constexpr int ln_threads(int lpr) { return lpr > 512 ? lpr : 512; }
 
 // Forward, row in registers: one read of x, one write of y; bound by HBM.
 // f32 [8192, 4096]: 46 us (5.8 TB/s) against 115 on the looping kernel, which
@@ -386,10 +386,10 @@ __device__ __forceinline__ void ln_bwd_load(const LnBwd<T>& a, const RowVec<T, L
     for (int e = 0; e < kVec<T>; ++e) xh[k][e] = (xh[k][e] - mu) * rs;
 }
 
-// dgamma and dbeta of 2 V columns over all rows (one workgroup of 256): 128
+// dgamma and dbeta of 2 V columns over all rows (one workgroup of 512): 256
 // row slots of two lanes, four rows in flight a slot, the slots added in LDS
 // by a fixed-order tree.
-constexpr int kLnColThreads = 256, kLnColLanes = 2, kLnColSlots = kLnColThreads / kLnColLanes;
+constexpr int kLnColThreads = 512, kLnColLanes = 2, kLnColSlots = kLnColThreads / kLnColLanes;
 template <typename T>
 constexpr int ln_col_lds() { return kLnColSlots * (2 * kLnColLanes * kVec<T> + 1); }  // floats
 template <typename T>
@@ -425,9 +425,22 @@ __device__ __forceinline__ void ln_bwd_columns(const LnBwd<T>& a, int block, flo
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) add(xv[u], dv[u], mu[u], rs[u]);
   }
-  for (; r < a.M; r += kLnColSlots) {
-    const int64_t at = (int64_t)r * a.N + c0;
-    add(*reinterpret_cast<const vec*>(a.x + at), *reinterpret_cast<const vec*>(a.dy + at), a.mean[r], a.rstd[r]);
+  if (r < a.M) {  // the rest in one batch too; rows past M read the last one and add zeros
+    vec xv[UNROLL - 1], dv[UNROLL - 1];
+    float mu[UNROLL - 1], rs[UNROLL - 1];
+#pragma unroll
+    for (int u = 0; u < UNROLL - 1; ++u) {
+      const bool on = r + u * kLnColSlots < a.M;
+      const int row = on ? r + u * kLnColSlots : a.M - 1;
+      const int64_t at = (int64_t)row * a.N + c0;
+      xv[u] = *reinterpret_cast<const vec*>(a.x + at);
+      dv[u] = *reinterpret_cast<const vec*>(a.dy + at);
+      mu[u] = a.mean[row];
+      rs[u] = a.rstd[row];
+      if (!on) xv[u] = dv[u] = vec{}, mu[u] = rs[u] = 0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < UNROLL - 1; ++u) add(xv[u], dv[u], mu[u], rs[u]);
   }
 #pragma unroll
   for (int e = 0; e < V; ++e) {
@@ -452,7 +465,7 @@ __device__ __forceinline__ void ln_bwd_columns(const LnBwd<T>& a, int block, flo
   }
 }
 
-// f16 [1500, 1000]: 8.8 us against 146 for a dx kernel and a column kernel of
+// f16 [1500, 1000]: 8.0 us against 146 for a dx kernel and a column kernel of
 // N / 64 workgroups that walk all rows.
 // Backward in one launch: the first `row_blocks` workgroups compute dx, a row
 // per LPR lanes; the others dgamma and dbeta, reading x and dy a second time,
@@ -703,11 +716,13 @@ Status ln_bwd_run(LnBwd<T> a, bool apart, hipStream_t s) {
   // Large matrices: x and dy read once, P chunks of rows (one workgroup per
   // CU), partial sums in dx.  Below 16 MiB (x and dy together an eighth of the
   // 256 MB MALL) the second read of the one-launch form comes from the caches
-  // and its two launches less count more; fewer than 8 rows a chunk would
-  // leave a quarter or more of the rows to the last launch.
+  // and its two launches less count more, until its N / 2 V column workgroups
+  // have too many rows each: f32 [2048, 632] 10.6 us against 13.9 fused,
+  // [4096, 512] 22.7 against 13.1, [16384, 100] 50 against 18.  Fewer than 8
+  // rows a chunk would leave a quarter or more of the rows to the last launch.
   constexpr int64_t kFusedBytes = 16 << 20;
-  constexpr int kChunks = 256;
-  if (apart && nv <= 2048 && M >= 8 * kChunks && (int64_t)M * N * (int64_t)sizeof(T) >= kFusedBytes) {
+  constexpr int kChunks = 256, kFusedRows = 3584;
+  if (apart && nv <= 2048 && M >= 8 * kChunks && ((int64_t)M * N * (int64_t)sizeof(T) >= kFusedBytes || M >= kFusedRows)) {
     a.P = kChunks;
     a.q = M / kChunks;
     a.r = M % kChunks;
@@ -727,7 +742,7 @@ Status ln_bwd_run(LnBwd<T> a, bool apart, hipStream_t s) {
     if (st != Status::Ok) return st;
     return rows((int64_t)a.P * a.RS, 0, true);
   }
-  if (!apart || nv > 1024) {  // two launches: dx may be x's or dy's memory, or its rows take wider workgroups
+  if (!apart || nv > 2048) {  // two launches: dx may be x's or dy's memory, or its rows take wider workgroups
     ln_bwd_columns_kernel<T><<<col_blocks, kLnColThreads, 0, s>>>(a);
     const Status st = launch_status("layernorm_bwd_columns");
     if (st != Status::Ok) return st;

@@ -223,7 +223,14 @@ __global__ __launch_bounds__(THREADS) void colsum_narrow_kernel(const TI* __rest
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) add_vec16<TI, BF16IN>(acc, q[u]);
     }
-    for (; r < M; r += SLOTS) add_vec16<TI, BF16IN>(acc, get(r));
+    if (r < M) {  // the rest in one batch too; rows past M read the last one and add zeros
+      uint4 q[UNROLL - 1];
+#pragma unroll
+      for (int u = 0; u < UNROLL - 1; ++u) q[u] = get(r + u * SLOTS < M ? r + u * SLOTS : M - 1);
+#pragma unroll
+      for (int u = 0; u < UNROLL - 1; ++u)
+        add_vec16<TI, BF16IN>(acc, r + u * SLOTS < M ? q[u] : uint4{0, 0, 0, 0});
+    }
   }
 #pragma unroll
   for (int e = 0; e < VEC; ++e) red[slot][v * VEC + e] = acc[e];

@@ -24,7 +24,7 @@ LN = [(1, 4, F32), (3, 5, F32), (2, 7, F32), (1, 8, F16), (3, 9, F16), (5, 15, F
       (3, 8191, F32), (2, 8193, F16), (2, 16384, F32), (2, 16385, F32), (1, 32768, F16), (300, 1000, F32),
       (1500, 264, F16),
       # the fused backward: 2048 rows, 16 MiB
-      (2048, 2048, F32), (2303, 2050, F32), (4097, 1025, F32), (2048, 8192, F32), (4300, 2049, F16),
+      (2048, 2048, F32), (3583, 24, F32), (3584, 9, F16), (5000, 33, F32), (2303, 2050, F32), (4097, 1025, F32), (2048, 8192, F32), (4300, 2049, F16),
       (2056, 4098, F16), (2049, 8200, F16), (16390, 516, F16)]
 
 
