@@ -1467,6 +1467,10 @@ Status run_gemm(GemmParams& p, hipStream_t s) {
       g.relu = p.act == ACT_RELU;
       if (small_gemm_ok(g)) return small_gemm_f32(g, s);
     }
+    // at most half a 64 x 64 tile a CU: K split over groups of waves (512 x
+    // 1024 x 4096 67 -> 46 us, 1856 x 184 x 3392 TN 54 -> 40)
+    const int64_t tiles64x32 = ((p.M + 63) / 64) * ((p.N + 31) / 32);
+    if (tiles64x32 <= 256 && p.K >= 512 && edge_gemm_ok(p, IN)) return edge_gemm(p, IN, OUT, s);
   }
   {
     constexpr bool MN = true;
@@ -1507,7 +1511,10 @@ Status run_gemm(GemmParams& p, hipStream_t s) {
     // 112.6 -> 19.8 us, fp32 1024^3 NN 53.8 -> 19.7 us against the
     // general-stride kernel)
     constexpr bool MN64 = true;
-    if (tiles128 >= 128 && nt_eligible<IN, OUT>(p, 128, 128, true)) {
+    // (fp32 is bound by its MFMAs, so by the tiles of the fullest CU: 2048 x
+    // 1024 x 512 33.4 us on 128 CUs with a 128 x 128 tile each, 18.9 on 64 x 64;
+    // 4096 x 512 x 1024 62.5, 33.5)
+    if (tiles128 >= (IN == IN_F32 ? 384 : 128) && nt_eligible<IN, OUT>(p, 128, 128, true)) {
       if constexpr (IN != IN_F32) {
         if (deep && tiles128 <= 256) return run_nt<IN, OUT, 128, 128, 2, 2, true, 4>(p, s);
       }
@@ -1515,10 +1522,11 @@ Status run_gemm(GemmParams& p, hipStream_t s) {
     }
     // at most one 32 x 32 tile a CU and K >= 2048: the edge kernel splits K
     // eight ways (64 x 256 x 4096 11.6 -> 9.7 us, 256 x 1024 x 4096 12.0 ->
-    // 10.5 against the 64 x 64 tiles with 8 stages)
+    // 10.5 against the 64 x 64 tiles with 8 stages; M-contiguous A from K =
+    // 4096: 256 x 256 x 8192 23.1 -> 17.5, 512 x 512 x 4096 equal)
     if constexpr (IN != IN_F32) {
       const int64_t tiles32 = ((p.M + 31) / 32) * ((p.N + 31) / 32);
-      if (tiles32 <= 256 && p.K >= 2048 && p.a_mode == LD_KCONTIG && edge_gemm_ok(p, IN))
+      if (tiles32 <= 256 && p.K >= (p.a_mode == LD_KCONTIG ? 2048 : 4096) && edge_gemm_ok(p, IN))
         return edge_gemm(p, IN, OUT, s);
     }
     // fewer tiles than CUs at 128x128: 64x64 tiles (4 waves of 32x32)

@@ -487,7 +487,9 @@ Status run_edge(const GemmParams& g, hipStream_t s) {
 //     without), four on 64 x 32 (f32 777 x 523 x 1000 15.5, 24.0), four on
 //     64 x 64 (640 x 1405 x 3128 NN 28.3, 46.7 without), each while it is at
 //     most one workgroup a CU;
-//   64 x 64 for short K: 6464 x 6377 x 18 38.7, 41.5 on 128 x 64, 65 on 256.
+//   short K: 64 x 128 from 7/8 of the CUs (4096 x 4394 x 64 15.1, 17.1 on 64 x
+//     64; 6464 x 6377 x 18 37.7, 39.9, 41.7 on 128 x 64, 65 on 256 x 256), else
+//     64 x 64.
 template <int IN, int OUT>
 Status run_edge_tiles(const GemmParams& g, hipStream_t s) {
   const int64_t nk = (g.K * (IN == IN_F32 ? 4 : 2) + 127) / 128;
@@ -502,6 +504,7 @@ Status run_edge_tiles(const GemmParams& g, hipStream_t s) {
     if (tiles(64, 32) <= 256) return run_edge<IN, OUT, 64, 32, 2, 1, 4, 1>(g, s);
     if (tiles(64, 64) <= 256) return run_edge<IN, OUT, 64, 64, 2, 2, 4, 1>(g, s);
   }
+  if (nk < 4 && tiles(64, 128) >= 224) return run_edge<IN, OUT, 64, 128, 2, 4, 1, 1>(g, s);
   return run_edge<IN, OUT, 64, 64, 2, 2, 1, 1>(g, s);
 }
 

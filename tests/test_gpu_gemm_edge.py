@@ -59,7 +59,9 @@ SIZES = [(1, 1, 8, 0, 0), (9, 3, 8, 1, 1), (64, 64, 9, 0, 0), (17, 10, 15, 3, 2)
          # K split 8 ways on 32 x 32, 4 ways on 64 x 32 and on 64 x 64 tiles
          (64, 10, 784, 0, 0), (33, 257, 1031, 1, 1), (500, 511, 523, 0, 0), (517, 700, 519, 1, 0),
          (650, 1000, 525, 0, 1), (1000, 1001, 1023, 0, 0),
+         (192, 256, 4160, 0, 0), (512, 1024, 576, 0, 0),  # the same where the tiles divide the shape
          (1030, 1029, 72, 0, 0), (2049, 520, 40, 1, 1),  # 64 x 64 tiles, short K
+         (2050, 1031, 40, 1, 1), (2048, 1024, 192, 0, 0),  # 64 x 128
          (2050, 1031, 265, 1, 1), (1100, 2051, 784, 0, 0),  # 128 x 64
          (2561, 2051, 255, 0, 0), (2600, 2500, 264, 8, 8),  # 128 x 128
          (3600, 3599, 520, 0, 0), (3333, 4099, 1000, 0, 1),  # 256 x 256
