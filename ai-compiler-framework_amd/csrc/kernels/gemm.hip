@@ -1332,9 +1332,9 @@ Status run_nt_layout(const GemmParams& g, hipStream_t s) {
     case ACT_GELU: return run_nt_act<IN, OUT, ACT_GELU, BM, BN, WM, WN, AKC, BKC, S>(g, s);
     case ACT_DGELU: return run_nt_act<IN, OUT, ACT_DGELU, BM, BN, WM, WN, AKC, BKC, S>(g, s);
     case ACT_ADAMW:
-      if constexpr (OUT == OUT_F32 && BM == 256 && BN == 256)
-        return run_nt_act<IN, OUT, ACT_ADAMW, BM, BN, WM, WN, AKC, BKC>(g, s);
-      return Status::Internal;  // fused AdamW runs on the 256 x 256 fp32-output tiles only
+      if constexpr (IN == IN_BF16 && OUT == OUT_F32)
+        return run_nt_act<IN, OUT, ACT_ADAMW, BM, BN, WM, WN, AKC, BKC, S>(g, s);
+      return Status::Internal;  // fused AdamW takes bf16 operands and an fp32 gradient
     default: return run_nt_act<IN, OUT, ACT_NONE, BM, BN, WM, WN, AKC, BKC, S>(g, s);
   }
 }
@@ -1422,20 +1422,81 @@ bool nt_eligible(const GemmParams& p, int BM, int BN, bool mn_ok) {
   return true;
 }
 
+// Column sums of a 256 x 256 block of a stored bf16 matrix, row t of
+// out [M/256, N] for block row t, in the order of the epilogue's
+// copy_out_colsum: a lane takes one 8-column chunk and every 16th row, lanes
+// l and l + 32 are added, then the 8 waves in order.
+__global__ __launch_bounds__(512) void tile_colsum_kernel(const uint16_t* __restrict__ c, int64_t ldc,
+                                                          float* __restrict__ out, int N) {
+  __shared__ float red[8][256];
+  const int tid = threadIdx.x, n0 = blockIdx.x * 256;
+  const uint16_t* src = c + ((int64_t)blockIdx.y * 256 + (tid >> 5)) * ldc + n0 + (tid & 31) * 8;
+  u16x8 x[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) x[k] = *reinterpret_cast<const u16x8*>(src + (int64_t)k * 16 * ldc);
+  float cs[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) cs[e] = 0.0f;
+#pragma unroll
+  for (int k = 0; k < 16; ++k)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) cs[e] += bf16_to_f32(x[k][e]);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) cs[e] += __shfl_xor(cs[e], 32, 64);
+  const int w = tid >> 6, l = tid & 63;
+  if (l < 32) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) red[w][l * 8 + e] = cs[e];
+  }
+  __syncthreads();
+  if (tid < 256) {
+    float s = red[0][tid];
+#pragma unroll
+    for (int k = 1; k < 8; ++k) s += red[k][tid];
+    out[(int64_t)blockIdx.y * N + n0 + tid] = s;
+  }
+}
+
 template <int IN, int OUT>
 Status run_gemm(GemmParams& p, hipStream_t s) {
-  if (p.colsum) {  // dGELU with column sums: the 8-wave 256 x 256 bf16-output path only
+  if (p.colsum) {  // dGELU with column sums, bf16 output, M and N multiples of 256
     if constexpr (OUT == OUT_BF16 && IN != IN_F32) {
-      // the column sums live in that configuration's epilogue (8 waves,
-      // whole tile in one pass): dispatch to it directly
-      if (p.act == ACT_DGELU && nt_eligible<IN, OUT>(p, 256, 256, true))
-        return run_nt<IN, OUT, 256, 256, 2, 4, true>(p, s);
+      if (p.act == ACT_DGELU && nt_eligible<IN, OUT>(p, 256, 256, true)) {
+        // the column sums live in the 8-wave 256 x 256 configuration's
+        // epilogue (whole tile in one pass): dispatch to it directly
+        if ((p.M / 256) * (p.N / 256) >= 128) return run_nt<IN, OUT, 256, 256, 2, 4, true>(p, s);
+        // fewer of those tiles than half the CUs: smaller ones, then the sums
+        // from the stored output, in the same order (256 x 3584 x 3584: 72 ->
+        // 21 us, 2048^3 49 -> 28; same bits)
+        float* colsum = p.colsum;
+        p.colsum = nullptr;
+        const Status st = run_gemm<IN, OUT>(p, s);
+        p.colsum = colsum;
+        if (st != Status::Ok) return st;
+        tile_colsum_kernel<<<dim3((unsigned)(p.N / 256), (unsigned)(p.M / 256)), 512, 0, s>>>(
+            (const uint16_t*)p.C, p.c_rs, colsum, (int)p.N);
+        return launch_status("gemm_tile_colsum");
+      }
     }
     return Status::NotImplemented;
   }
-  if (p.act == ACT_ADAMW) {  // the fused optimizer epilogue exists on the 256 x 256 NT path only
+  if (p.act == ACT_ADAMW) {  // the fused optimizer epilogue: M and N multiples of 256
     if constexpr (OUT == OUT_F32 && IN == IN_BF16) {
-      if (nt_eligible<IN, OUT>(p, 256, 256, true)) return run_nt256<IN, OUT>(p, s);
+      if (nt_eligible<IN, OUT>(p, 256, 256, true)) {
+        // the largest tiles that give every other CU one, as for the other
+        // epilogues (the gradient's bits are the same: K order does not depend
+        // on the tile): 1024 x 1024 x 8192 174 -> 37 us, 2048 x 2048 x 8192 181
+        // -> 85, 2560 x 2560 x 4096 122 -> 87 (400 tiles of 128 x 128)
+        const int64_t tiles128 = (p.M / 128) * (p.N / 128);
+        const bool deep = p.K >= 16 * 64;
+        if (tiles128 >= 512) return run_nt256<IN, OUT>(p, s);
+        if (tiles128 >= 128) {
+          if (deep && tiles128 <= 256) return run_nt<IN, OUT, 128, 128, 2, 2, true, 4>(p, s);
+          return run_nt<IN, OUT, 128, 128, 2, 2, true>(p, s);
+        }
+        if (deep) return run_nt<IN, OUT, 64, 64, 2, 2, true, 8>(p, s);
+        return run_nt<IN, OUT, 64, 64, 2, 2, true>(p, s);
+      }
     }
     return Status::NotImplemented;
   }
@@ -1651,8 +1712,8 @@ bool epi_check(const TensorDesc* in, int ni, const TensorDesc* out, int no, cons
         W.shape[0] < C.rows / 256)
       return false;
     if (!fin && W.shape[0] != C.rows / 256) return false;  // its reader sums every row
-    // only the bf16 256 x 256-tile path carries the column sums: accept
-    // exactly the calls it runs (M, N multiples of 256, so the workspace
+    // the column sums are kept per 256-row block: accept exactly the calls
+    // that run_gemm takes with them (M, N multiples of 256, so the workspace
     // has at least one row; K of 64; aligned operands)
     if (din != DType::kBF16) return false;
     GemmParams p{};
@@ -1660,6 +1721,8 @@ bool epi_check(const TensorDesc* in, int ni, const TensorDesc* out, int no, cons
     p.act = ACT_DGELU;
     p.aux = const_cast<void*>(X.data);
     p.aux_rs = X.stride[0];
+    p.colsum = (float*)W.data;
+    if (!p.colsum) return false;
     return nt_eligible<IN_BF16, OUT_BF16>(p, 256, 256, true);
   }
   if (no > 2) return false;
@@ -1746,9 +1809,8 @@ EPI_VARIANT(epi_bf16_f32out, DType::kBF16, DType::kF32, false)
 // to memory.  inputs (A bf16, B bf16, P f32, M f32, V f32, step i32 scalar),
 // outputs (P, M, V in place, Wb bf16 shadow of P); P, M, V, Wb are [M, N]
 // row-major views; grad = op(A) . op(B).  Attr schema GADW
-// <ii fffff>: transA, transB, lr, beta1, beta2, eps, weight_decay.  Only the
-// 256 x 256-tile path carries this epilogue (bf16 operands, M and N
-// multiples of 256, K of 64, 16-byte aligned rows); other shapes are not
+// <ii fffff>: transA, transB, lr, beta1, beta2, eps, weight_decay.  M and N
+// multiples of 256, K of 64, 16-byte aligned rows; other shapes are not
 // supported.
 // ---------------------------------------------------------------------------
 struct GadwAttr {
