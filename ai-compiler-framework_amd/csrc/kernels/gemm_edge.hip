@@ -514,9 +514,9 @@ bool edge_gemm_ok(const GemmParams& p, int in) {
   const int64_t es = in == IN_F32 ? 4 : 2, ce = 16 / es;
   if (p.colsum || p.act == ACT_ADAMW || p.c_cs != 1) return false;
   if (p.M > INT32_MAX / 2 || p.N > INT32_MAX / 2 || p.K > INT32_MAX / 2 || p.K < ce) return false;
-  // 32-bit offsets from a tile's first row, for 128 rows of it
+  // 32-bit offsets from a tile's first row, for the up to 256 rows of it
   auto operand_ok = [&](int mode, int64_t ld_k, int64_t ld_mn, int64_t mn) {
-    if (mode == LD_KCONTIG) return 128 * ld_k * es < INT32_MAX;
+    if (mode == LD_KCONTIG) return 256 * ld_k * es < INT32_MAX;
     return mode == LD_MNCONTIG && mn >= ce && 128 * ld_mn * es < INT32_MAX;
   };
   if (!operand_ok(p.a_mode, p.a_rs, p.a_cs, p.M) || !operand_ok(p.b_mode, p.b_cs, p.b_rs, p.N)) return false;
