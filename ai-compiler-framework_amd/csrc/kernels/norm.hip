@@ -673,33 +673,50 @@ Status ln_fwd_run(const T* x, const T* g, const T* b, T* y, float* mean, float* 
   return launch_status("layernorm_fwd");
 }
 
-// Whether the call may use dx for partial sums and write dx rows before other
-// rows of x and dy have been read: dx shares no byte with an input or another
-// output.
-bool ln_dx_apart(const TensorDesc* in, int ni, const TensorDesc* out, int no) {
-  for (int k = 0; k < ni; ++k)
-    if (views_overlap(out[0], in[k])) return false;
-  for (int k = 1; k < no; ++k)
-    if (views_overlap(out[0], out[k])) return false;
+// Whether out[k] shares no byte with an input or another output.
+bool output_apart(const TensorDesc* in, int ni, const TensorDesc* out, int no, int k) {
+  for (int i = 0; i < ni; ++i)
+    if (views_overlap(out[k], in[i])) return false;
+  for (int i = 0; i < no; ++i)
+    if (i != k && views_overlap(out[k], out[i])) return false;
   return true;
 }
 
+// What a backward call's outputs allow.  Apart: dx may hold partial sums, and
+// its rows may be written before other rows of x and dy have been read.
+// OnDx: dx is x's or dy's memory.  OnSums: dgamma or dbeta is memory that the
+// call reads or dx (an input may be given up for them): dx is complete before
+// they are written.
+enum class LnOut { Apart, OnDx, OnSums };
+LnOut ln_bwd_outputs(const TensorDesc* in, int ni, const TensorDesc* out, int no) {
+  for (int k = 1; k < no; ++k)
+    if (!output_apart(in, ni, out, no, k)) return LnOut::OnSums;
+  return output_apart(in, ni, out, no, 0) ? LnOut::Apart : LnOut::OnDx;
+}
+
 template <typename T>
-Status ln_bwd_run(LnBwd<T> a, bool apart, hipStream_t s) {
+Status ln_bwd_run(LnBwd<T> a, LnOut where, hipStream_t s) {
   constexpr int V = kVec<T>;
   const int M = a.M, N = a.N;
   const int64_t nv = ((int64_t)N + V - 1) / V;
   const bool affine = a.dgamma != nullptr;
+  auto sums_loop = [&] {
+    ln_bwd_dgdb_loop_kernel<T><<<(unsigned)(((int64_t)N + 63) / 64), 256, 0, s>>>(a.x, a.dy, a.mean, a.rstd,
+                                                                                a.dgamma, a.dbeta, M, N);
+    return launch_status("layernorm_bwd_dgdb");
+  };
+  auto in_order = [&](auto first, auto second) {
+    const Status st = first();
+    return st == Status::Ok ? second() : st;
+  };
   if (N < V || nv > kLnMaxVecs) {
-    if (affine) {  // before dx, which may be x's or dy's own memory
-      ln_bwd_dgdb_loop_kernel<T><<<(unsigned)(((int64_t)N + 63) / 64), 256, 0, s>>>(a.x, a.dy, a.mean, a.rstd,
-                                                                                  a.dgamma, a.dbeta, M, N);
-      const Status st = launch_status("layernorm_bwd_dgdb");
-      if (st != Status::Ok) return st;
-    }
-    ln_bwd_dx_loop_kernel<T><<<(unsigned)(((int64_t)M + 3) / 4), 256, 0, s>>>(a.x, a.dy, a.gamma, a.mean, a.rstd,
-                                                                              a.dx, M, N);
-    return launch_status("layernorm_bwd");
+    auto dx_loop = [&] {
+      ln_bwd_dx_loop_kernel<T><<<(unsigned)(((int64_t)M + 3) / 4), 256, 0, s>>>(a.x, a.dy, a.gamma, a.mean, a.rstd,
+                                                                                a.dx, M, N);
+      return launch_status("layernorm_bwd");
+    };
+    if (!affine) return dx_loop();
+    return where == LnOut::OnSums ? in_order(dx_loop, sums_loop) : in_order(sums_loop, dx_loop);
   }
   const unsigned col_blocks = (unsigned)((nv + kLnColLanes - 1) / kLnColLanes);
   auto rows = [&](int64_t n, unsigned extra, bool reserved) {
@@ -712,7 +729,11 @@ Status ln_bwd_run(LnBwd<T> a, bool apart, hipStream_t s) {
 #undef LN_BWD
     return launch_status("layernorm_bwd");
   };
-  if (!affine) return rows(M, 0, false);
+  auto all_rows = [&] { return rows(M, 0, false); };
+  if (!affine) return all_rows();
+  // dx, then the sums, 64 columns a workgroup (which has read all of them when
+  // it writes): the sums may lie on gamma, and at N <= 64 on any input
+  if (where == LnOut::OnSums) return in_order(all_rows, sums_loop);
   // Large matrices: x and dy read once, P chunks of rows (one workgroup per
   // CU), partial sums in dx.  Below 16 MiB (x and dy together an eighth of the
   // 256 MB MALL) the second read of the one-launch form comes from the caches
@@ -722,7 +743,7 @@ Status ln_bwd_run(LnBwd<T> a, bool apart, hipStream_t s) {
   // rows a chunk would leave a quarter or more of the rows to the last launch.
   constexpr int64_t kFusedBytes = 16 << 20;
   constexpr int kChunks = 256, kFusedRows = 3584;
-  if (apart && nv <= 2048 && M >= 8 * kChunks && ((int64_t)M * N * (int64_t)sizeof(T) >= kFusedBytes || M >= kFusedRows)) {
+  if (where == LnOut::Apart && nv <= 2048 && M >= 8 * kChunks && ((int64_t)M * N * (int64_t)sizeof(T) >= kFusedBytes || M >= kFusedRows)) {
     a.P = kChunks;
     a.q = M / kChunks;
     a.r = M % kChunks;
@@ -742,11 +763,12 @@ Status ln_bwd_run(LnBwd<T> a, bool apart, hipStream_t s) {
     if (st != Status::Ok) return st;
     return rows((int64_t)a.P * a.RS, 0, true);
   }
-  if (!apart || nv > 2048) {  // two launches: dx may be x's or dy's memory, or its rows take wider workgroups
-    ln_bwd_columns_kernel<T><<<col_blocks, kLnColThreads, 0, s>>>(a);
-    const Status st = launch_status("layernorm_bwd_columns");
-    if (st != Status::Ok) return st;
-    return rows(M, 0, false);
+  if (where == LnOut::OnDx || nv > 2048) {  // two launches: the sums before dx, or its rows take wider workgroups
+    auto columns = [&] {
+      ln_bwd_columns_kernel<T><<<col_blocks, kLnColThreads, 0, s>>>(a);
+      return launch_status("layernorm_bwd_columns");
+    };
+    return in_order(columns, all_rows);
   }
   return rows(M, col_blocks, false);
 }
@@ -782,7 +804,7 @@ Status ln_bwd_run(LnBwd<T> a, bool apart, hipStream_t s) {
     b.dbeta = aff ? (float*)o[2].data : nullptr;                                                       \
     b.M = (int)i[0].shape[0];                                                                          \
     b.N = (int)i[0].shape[1];                                                                          \
-    return ln_bwd_run<T>(b, ln_dx_apart(i, ni, o, no), as_stream(s));                                  \
+    return ln_bwd_run<T>(b, ln_bwd_outputs(i, ni, o, no), as_stream(s));                               \
   }
 
 LN_VARIANTS(f32, float, DType::kF32)
