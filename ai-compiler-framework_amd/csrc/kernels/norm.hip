@@ -1198,8 +1198,8 @@ __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const uint16_t* x,
   }
 }
 
-// Channels too large for registers whose output cannot hold the partial sums
-// (it shares memory with an input): one workgroup a channel, x read from
+// Channels too large for registers that cannot be split over workgroups (an
+// output shares memory with an input): one workgroup a channel, x read from
 // memory for each pass.
 __device__ __forceinline__ int64_t bn_index(const BNShape& s, int c, int64_t k) {
   const int64_t n = k / s.HW, hw = k - n * s.HW;
@@ -1259,13 +1259,14 @@ __global__ __launch_bounds__(256) void bn_bwd_loop_kernel(const uint16_t* x, con
   }
 }
 
-// Whether the output may hold partial sums while the inputs are still read:
-// it shares no byte with an input or another output.
-bool bn_out_apart(const TensorDesc* in, int ni, const TensorDesc* out, int no) {
-  for (int k = 0; k < ni; ++k)
-    if (views_overlap(out[0], in[k])) return false;
-  for (int k = 1; k < no; ++k)
-    if (views_overlap(out[0], out[k])) return false;
+// Whether a channel may be split over workgroups and kernels: the large output
+// holds partial sums while the inputs are read, and the per-channel outputs
+// are written by one kernel and read by the next, so none of them shares a
+// byte with an input or another output.  (One workgroup a channel reads all
+// that it needs of its channel before it writes.)
+bool bn_outputs_apart(const TensorDesc* in, int ni, const TensorDesc* out, int no) {
+  for (int k = 0; k < no; ++k)
+    if (!output_apart(in, ni, out, no, k)) return false;
   return true;
 }
 
@@ -1406,7 +1407,7 @@ Status bn_fwd_launch(const TensorDesc* in, int ni, TensorDesc* out, int no, cons
     const uint16_t* g = ni == 3 ? (const uint16_t*)in[1].data : nullptr;
     const uint16_t* b = ni == 3 ? (const uint16_t*)in[2].data : nullptr;
     float *sm = (float*)out[1].data, *sr = (float*)out[2].data;
-    const bool apart = bn_out_apart(in, ni, out, no);
+    const bool apart = bn_outputs_apart(in, ni, out, no);
     if (sh.HW % 8 == 0) return bn_fwd_train<8>(x, g, b, y, sm, sr, sh, A.eps, apart, s);
     if (sh.HW % 4 == 0) return bn_fwd_train<4>(x, g, b, y, sm, sr, sh, A.eps, apart, s);
     return bn_fwd_train<1>(x, g, b, y, sm, sr, sh, A.eps, apart, s);
@@ -1447,7 +1448,7 @@ Status bn_bwd_launch(const TensorDesc* in, int ni, TensorDesc* out, int no, cons
   const float *sm = (const float*)in[3].data, *sr = (const float*)in[4].data;
   uint16_t* dx = (uint16_t*)out[0].data;
   float *dg = (float*)out[1].data, *db = (float*)out[2].data;
-  const bool apart = bn_out_apart(in, ni, out, no);
+  const bool apart = bn_outputs_apart(in, ni, out, no);
   hipStream_t s = as_stream(stream);
   if (sh.HW % 8 == 0) return bn_bwd_run<8>(x, dy, g, sm, sr, dx, dg, db, sh, apart, s);
   if (sh.HW % 4 == 0) return bn_bwd_run<4>(x, dy, g, sm, sr, dx, dg, db, sh, apart, s);

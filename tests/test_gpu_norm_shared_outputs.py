@@ -1,6 +1,6 @@
-"""GPU parity of the normalisation backward where its sums are written over
-memory that the same call reads (gamma, the saved statistics, the input), for
-every form of the call; against the fp64 oracle on the inputs as they were,
+"""GPU parity of the normalisations where their sums are written over memory
+that the same call reads (gamma, the saved statistics, the input), for every
+form of the call; against the fp64 oracle on the inputs as they were,
 with test_gpu_norm.py's tolerances (fp32 1e-5, f16 2e-3)."""
 from __future__ import annotations
 
@@ -56,3 +56,23 @@ def test_layernorm_sums_over_what_one_workgroup_reads(C, n, onto):
     outs = [torch.empty_like(x)] + ([mean, rstd] if onto == "statistics" else [x[0], dy[n - 1]])
     C.op_call(C.OpKind.LayerNormBwd, [x, dy, g, mean, rstd], outs)
     assert check_ln([x], outs)(ref)
+
+
+# a channel in registers; split over workgroups, in vectors of 8, 4 and 1
+BN = [(4, 5, 8, 8), (32, 6, 56, 56), (83, 3, 28, 28), (180, 2, 14, 14), (200, 3, 7, 7)]
+
+
+@pytest.mark.parametrize("shape", BN)
+@pytest.mark.parametrize("dx_on", [None, "x", "dy"])
+def test_batchnorm_sums_over_the_saved_statistics(C, shape, dx_on):
+    r = rng(sum(shape))
+    Cc = shape[1]
+    x, dy = dev(r.standard_normal(shape) * 1.5 + 0.25, F16), dev(r.standard_normal(shape), F16)
+    g = dev(r.standard_normal(Cc), F16)
+    x64 = host(x)
+    mean, rstd = dev(x64.mean((0, 2, 3)), F32), dev(1 / (x64.var((0, 2, 3)) + 1e-5) ** 0.5, F32)
+    ref = orc.batchnorm_bwd_f64(x64, host(dy), host(g), host(mean), host(rstd))
+    dx = {None: torch.empty_like(x), "x": x, "dy": dy}[dx_on]
+    C.op_call(C.OpKind.BatchNormBwd, [x, dy, g, mean, rstd], [dx, mean, rstd])
+    assert orc.rel_err(host(dx), ref[0]) < 2e-3
+    assert orc.rel_err(host(mean), ref[1]) < 1e-5 and orc.rel_err(host(rstd), ref[2]) < 1e-5
