@@ -66,36 +66,37 @@ __device__ __forceinline__ void st_from_f32(T* p, int64_t i, float v) {
 // ===========================================================================
 // LayerNorm
 // ===========================================================================
-// Any N, one wave per row, the row read two or three times: rows shorter than
-// a vector or longer than the register-resident kernels hold.
+// Any M and N, one wave per row (and every gridDim.x * 4 th row on), the row
+// read two or three times: rows shorter than a vector or longer than the
+// register-resident kernels hold, and more rows than one launch has lanes for.
 template <typename T>
 __global__ __launch_bounds__(256) void ln_fwd_loop_kernel(const T* x, const T* gamma,
                                                           const T* beta, T* y,
                                                           float* mean, float* rstd,
                                                           int M, int N, float eps) {
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= M) return;  // whole wave
-  const T* xr = x + (int64_t)row * N;
-  T* yr = y + (int64_t)row * N;
   const float invN = 1.0f / (float)N;
-  float s = 0.0f;
-  for (int c = lane; c < N; c += 64) s += ld_as_f32(xr, c);
-  const float mu = wave_sum(s) * invN;
-  float d = 0.0f;
-  for (int c = lane; c < N; c += 64) {
-    const float t = ld_as_f32(xr, c) - mu;
-    d = fmaf(t, t, d);
-  }
-  const float rs = 1.0f / sqrtf(wave_sum(d) * invN + eps);
-  for (int c = lane; c < N; c += 64) {
-    float o = (ld_as_f32(xr, c) - mu) * rs;
-    if (gamma) o = fmaf(o, ld_as_f32(gamma, c), ld_as_f32(beta, c));
-    st_from_f32(yr, c, o);
-  }
-  if (lane == 0) {
-    mean[row] = mu;
-    rstd[row] = rs;
+  for (int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); row < M; row += (int64_t)gridDim.x * 4) {
+    const T* xr = x + row * N;
+    T* yr = y + row * N;
+    float s = 0.0f;
+    for (int c = lane; c < N; c += 64) s += ld_as_f32(xr, c);
+    const float mu = wave_sum(s) * invN;
+    float d = 0.0f;
+    for (int c = lane; c < N; c += 64) {
+      const float t = ld_as_f32(xr, c) - mu;
+      d = fmaf(t, t, d);
+    }
+    const float rs = 1.0f / sqrtf(wave_sum(d) * invN + eps);
+    for (int c = lane; c < N; c += 64) {
+      float o = (ld_as_f32(xr, c) - mu) * rs;
+      if (gamma) o = fmaf(o, ld_as_f32(gamma, c), ld_as_f32(beta, c));
+      st_from_f32(yr, c, o);
+    }
+    if (lane == 0) {
+      mean[row] = mu;
+      rstd[row] = rs;
+    }
   }
 }
 
@@ -108,28 +109,29 @@ __global__ __launch_bounds__(256) void ln_bwd_dx_loop_kernel(const T* x, const T
                                                              const float* rstd, T* dx,
                                                              int M, int N) {
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= M) return;
-  const T* xr = x + (int64_t)row * N;
-  const T* dyr = dy + (int64_t)row * N;
-  T* dxr = dx + (int64_t)row * N;
-  const float mu = mean[row], rs = rstd[row];
-  const float fN = (float)N, scale = rs / fN;
-  float s1 = 0.0f, s2 = 0.0f;
-  for (int c = lane; c < N; c += 64) {
-    const float xh = (ld_as_f32(xr, c) - mu) * rs;
-    float g = ld_as_f32(dyr, c);
-    if (gamma) g *= ld_as_f32(gamma, c);
-    s1 += g;
-    s2 = fmaf(g, xh, s2);
-  }
-  s1 = wave_sum(s1);
-  s2 = wave_sum(s2);
-  for (int c = lane; c < N; c += 64) {
-    const float xh = (ld_as_f32(xr, c) - mu) * rs;
-    float g = ld_as_f32(dyr, c);
-    if (gamma) g *= ld_as_f32(gamma, c);
-    st_from_f32(dxr, c, (fN * g - s1 - xh * s2) * scale);
+  const float fN = (float)N;
+  for (int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); row < M; row += (int64_t)gridDim.x * 4) {
+    const T* xr = x + row * N;
+    const T* dyr = dy + row * N;
+    T* dxr = dx + row * N;
+    const float mu = mean[row], rs = rstd[row];
+    const float scale = rs / fN;
+    float s1 = 0.0f, s2 = 0.0f;
+    for (int c = lane; c < N; c += 64) {
+      const float xh = (ld_as_f32(xr, c) - mu) * rs;
+      float g = ld_as_f32(dyr, c);
+      if (gamma) g *= ld_as_f32(gamma, c);
+      s1 += g;
+      s2 = fmaf(g, xh, s2);
+    }
+    s1 = wave_sum(s1);
+    s2 = wave_sum(s2);
+    for (int c = lane; c < N; c += 64) {
+      const float xh = (ld_as_f32(xr, c) - mu) * rs;
+      float g = ld_as_f32(dyr, c);
+      if (gamma) g *= ld_as_f32(gamma, c);
+      st_from_f32(dxr, c, (fN * g - s1 - xh * s2) * scale);
+    }
   }
 }
 
@@ -146,9 +148,9 @@ __global__ __launch_bounds__(256) void ln_bwd_dgdb_loop_kernel(const T* __restri
   const int c = blockIdx.x * 64 + lane;
   float sg = 0.0f, sb = 0.0f;
   if (c < N) {
-    for (int r = w; r < M; r += 4) {
-      const float xh = (ld_as_f32(x, (int64_t)r * N + c) - mean[r]) * rstd[r];
-      const float d = ld_as_f32(dy, (int64_t)r * N + c);
+    for (int64_t r = w; r < M; r += 4) {
+      const float xh = (ld_as_f32(x, r * N + c) - mean[r]) * rstd[r];
+      const float d = ld_as_f32(dy, r * N + c);
       sb += d;
       sg = fmaf(d, xh, sg);
     }
@@ -657,12 +659,23 @@ bool ln_bwd_check(const TensorDesc* in, int ni, const TensorDesc* out, int no, D
   else CALL(1024, 4)
 constexpr int kLnMaxVecs = 4096;  // longer rows take the looping kernels
 
+// Whether rows of nv vectors fit the register-resident kernels, and whether M
+// of them fit one launch: the runtime counts a grid's lanes in 32 bits and
+// starts too few workgroups, without an error, above that.
+constexpr bool ln_row_fits(int64_t N, int64_t nv, int V) { return N >= V && nv <= kLnMaxVecs; }
+constexpr bool ln_grid_fits(int64_t M, int64_t nv) {
+  int64_t lanes = 64;
+  while (nv > 4 * lanes) lanes *= 2;
+  return M * lanes <= (int64_t)UINT32_MAX - 1024;
+}
+unsigned ln_loop_blocks(int64_t M) { return (unsigned)((M + 3) / 4 < 1 << 22 ? (M + 3) / 4 : 1 << 22); }
+
 template <typename T>
 Status ln_fwd_run(const T* x, const T* g, const T* b, T* y, float* mean, float* rstd, int M, int N, float eps,
                   hipStream_t s) {
   const int64_t nv = ((int64_t)N + kVec<T> - 1) / kVec<T>;
-  if (N < kVec<T> || nv > kLnMaxVecs) {
-    ln_fwd_loop_kernel<T><<<(unsigned)(((int64_t)M + 3) / 4), 256, 0, s>>>(x, g, b, y, mean, rstd, M, N, eps);
+  if (!ln_row_fits(N, nv, kVec<T>) || !ln_grid_fits(M, nv)) {
+    ln_fwd_loop_kernel<T><<<ln_loop_blocks(M), 256, 0, s>>>(x, g, b, y, mean, rstd, M, N, eps);
     return launch_status("layernorm_fwd");
   }
 #define LN_FWD(LPR, VPT)                                                                                   \
@@ -700,6 +713,7 @@ Status ln_bwd_run(LnBwd<T> a, LnOut where, hipStream_t s) {
   const int M = a.M, N = a.N;
   const int64_t nv = ((int64_t)N + V - 1) / V;
   const bool affine = a.dgamma != nullptr;
+  const bool regs = ln_row_fits(N, nv, V), fits = regs && ln_grid_fits(M, nv);
   auto sums_loop = [&] {
     ln_bwd_dgdb_loop_kernel<T><<<(unsigned)(((int64_t)N + 63) / 64), 256, 0, s>>>(a.x, a.dy, a.mean, a.rstd,
                                                                                 a.dgamma, a.dbeta, M, N);
@@ -709,15 +723,6 @@ Status ln_bwd_run(LnBwd<T> a, LnOut where, hipStream_t s) {
     const Status st = first();
     return st == Status::Ok ? second() : st;
   };
-  if (N < V || nv > kLnMaxVecs) {
-    auto dx_loop = [&] {
-      ln_bwd_dx_loop_kernel<T><<<(unsigned)(((int64_t)M + 3) / 4), 256, 0, s>>>(a.x, a.dy, a.gamma, a.mean, a.rstd,
-                                                                                a.dx, M, N);
-      return launch_status("layernorm_bwd");
-    };
-    if (!affine) return dx_loop();
-    return where == LnOut::OnSums ? in_order(dx_loop, sums_loop) : in_order(sums_loop, dx_loop);
-  }
   const unsigned col_blocks = (unsigned)((nv + kLnColLanes - 1) / kLnColLanes);
   auto rows = [&](int64_t n, unsigned extra, bool reserved) {
 #define LN_BWD(LPR, VPT)                                                                                 \
@@ -729,11 +734,17 @@ Status ln_bwd_run(LnBwd<T> a, LnOut where, hipStream_t s) {
 #undef LN_BWD
     return launch_status("layernorm_bwd");
   };
-  auto all_rows = [&] { return rows(M, 0, false); };
-  if (!affine) return all_rows();
+  auto dx_all = [&] {
+    if (fits) return rows(M, 0, false);
+    ln_bwd_dx_loop_kernel<T><<<ln_loop_blocks(M), 256, 0, s>>>(a.x, a.dy, a.gamma, a.mean, a.rstd, a.dx, M, N);
+    return launch_status("layernorm_bwd");
+  };
+  if (!affine || M < 1) return dx_all();  // no rows: refused as an empty grid
   // dx, then the sums, 64 columns a workgroup (which has read all of them when
   // it writes): the sums may lie on gamma, and at N <= 64 on any input
-  if (where == LnOut::OnSums) return in_order(all_rows, sums_loop);
+  if (where == LnOut::OnSums) return in_order(dx_all, sums_loop);
+  // the kernels below step 32-bit row indices to less than 1024 past M
+  if (!regs || M > INT32_MAX - 1024) return in_order(sums_loop, dx_all);
   // Large matrices: x and dy read once, P chunks of rows (one workgroup per
   // CU), partial sums in dx.  Below 16 MiB (x and dy together an eighth of the
   // 256 MB MALL) the second read of the one-launch form comes from the caches
@@ -763,12 +774,12 @@ Status ln_bwd_run(LnBwd<T> a, LnOut where, hipStream_t s) {
     if (st != Status::Ok) return st;
     return rows((int64_t)a.P * a.RS, 0, true);
   }
-  if (where == LnOut::OnDx || nv > 2048) {  // two launches: the sums before dx, or its rows take wider workgroups
+  if (where == LnOut::OnDx || nv > 2048 || !fits) {  // two launches: the sums before dx, or its rows take other workgroups
     auto columns = [&] {
       ln_bwd_columns_kernel<T><<<col_blocks, kLnColThreads, 0, s>>>(a);
       return launch_status("layernorm_bwd_columns");
     };
-    return in_order(columns, all_rows);
+    return in_order(columns, dx_all);
   }
   return rows(M, col_blocks, false);
 }

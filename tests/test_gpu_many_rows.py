@@ -1,0 +1,68 @@
+"""GPU parity where a grid's lanes pass 2^32, which the runtime counts in 32
+bits: every row must still be computed.  The rows repeat a short pattern, whose
+result the fp64 oracle gives (fp32, normwise 1e-5); every repetition has the
+pattern's own bits."""
+from __future__ import annotations
+
+import struct
+
+import pytest
+import torch
+
+import oracle as orc
+from test_gpu_norm import LNEP, dev, host, rng
+
+pytestmark = pytest.mark.gpu
+
+
+def repeated(pattern, times):
+    return pattern.repeat(times, *([1] * (pattern.dim() - 1)))
+
+
+def same(t, n):
+    """Every n rows of t are its first n."""
+    v = t.view(-1, n, *t.shape[1:])
+    return all(bool((c == v[:1]).all()) for c in v.split(1 << 21))
+
+
+@pytest.mark.parametrize("N", [3, 8])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_layernorm_of_more_rows_than_a_grid(C, N, in_place):
+    n, times = 8, (1 << 23) + 1  # 2^26 + 8 rows, 64 lanes each
+    M = n * times
+    r = rng(N)
+    px, pdy = dev(r.standard_normal((n, N)) * 2 + 0.5, torch.float32), dev(r.standard_normal((n, N)), torch.float32)
+    g, b = dev(r.standard_normal(N), torch.float32), dev(r.standard_normal(N), torch.float32)
+    x, dy = repeated(px, times), repeated(pdy, times)
+    mean, rstd = torch.zeros(M, device="cuda"), torch.zeros(M, device="cuda")
+    y = x if in_place else torch.zeros_like(x)
+    C.op_call(C.OpKind.LayerNormFwd, [x, g, b], [y, mean, rstd], LNEP, struct.pack("<f", 1e-5))
+    y_ref, mu_ref, rs_ref = orc.layernorm_fwd_f64(host(px), host(g), host(b), eps=1e-5)
+    for got, want in ((y, y_ref), (mean, mu_ref), (rstd, rs_ref)):
+        assert orc.rel_err(host(got[:n]), want) < 1e-5 and same(got, n)
+    x.copy_(repeated(px, times))
+    dx_ref, dg_ref, db_ref = orc.layernorm_bwd_f64(host(px), host(pdy), mu_ref, rs_ref, host(g))
+    for affine in (False, True):
+        d = dy.clone()
+        dx = d if in_place else torch.zeros_like(x)
+        dg, db = torch.zeros(N, device="cuda"), torch.zeros(N, device="cuda")
+        if affine:
+            C.op_call(C.OpKind.LayerNormBwd, [x, d, g, mean, rstd], [dx, dg, db])
+            assert orc.rel_err(host(dx[:n]), dx_ref) < 1e-5
+            if N == 8:  # a lane adds up to 2^18 terms, each with an error of at most 2^-24 of the sum
+                tol = 2.0 ** -6
+                assert orc.rel_err(host(dg) / times, dg_ref) < tol and orc.rel_err(host(db) / times, db_ref) < tol
+        else:
+            C.op_call(C.OpKind.LayerNormBwd, [x, d, mean, rstd], [dx])
+        assert same(dx, n)
+
+
+@pytest.mark.parametrize("affine", [False, True])
+def test_layernorm_of_no_rows_is_refused(C, affine):
+    x, s, g = torch.empty((0, 8), device="cuda"), torch.empty(0, device="cuda"), torch.ones(8, device="cuda")
+    with pytest.raises(RuntimeError, match="Internal"):
+        if affine:
+            C.op_call(C.OpKind.LayerNormBwd, [x, x, g, s, s],
+                      [torch.empty_like(x), torch.empty(8, device="cuda"), torch.empty(8, device="cuda")])
+        else:
+            C.op_call(C.OpKind.LayerNormBwd, [x, x, s, s], [torch.empty_like(x)])
