@@ -745,6 +745,25 @@ template <int MODE>
 Status launch_rows(const RowArgs& a, void* stream) {
   hipStream_t s = as_stream(stream);
   const int64_t R = a.R, C = a.C;
+  // The runtime counts a grid's lanes in 32 bits and starts too few
+  // workgroups, without an error, above that; a row has at most 512.
+  constexpr int64_t kRows = (int64_t{1} << 23) - 16;
+  if (R > kRows) {
+    RowArgs part = a;
+    for (int64_t r = 0; r < R; r += kRows) {
+      part.R = R - r < kRows ? R - r : kRows;
+      part.x = a.x + r * C;
+      if (a.y) part.y = a.y + r * C;
+      if (a.rmax) part.rmax = a.rmax + r;
+      if (a.rsum) part.rsum = a.rsum + r;
+      if (a.labels) part.labels = a.labels + r;
+      if (a.argmax) part.argmax = a.argmax + r;
+      if (a.row_loss) part.row_loss = a.row_loss + r;
+      const Status st = launch_rows<MODE>(part, stream);
+      if (st != Status::Ok) return st;
+    }
+    return Status::Ok;
+  }
   const bool al = aligned(a.x, 16) && (a.y == nullptr || aligned(a.y, 16));
 #define ROW_CASE(LPR, VPT)                                                                  \
   if (al && C == (int64_t)(LPR) * (VPT) * 4) {                                               \

@@ -6,6 +6,7 @@ from __future__ import annotations
 
 import struct
 
+import numpy as np
 import pytest
 import torch
 
@@ -13,6 +14,8 @@ import oracle as orc
 from test_gpu_norm import LNEP, dev, host, rng
 
 pytestmark = pytest.mark.gpu
+
+RRED = int.from_bytes(b"RRED", "little")
 
 
 def repeated(pattern, times):
@@ -66,3 +69,35 @@ def test_layernorm_of_no_rows_is_refused(C, affine):
                       [torch.empty_like(x), torch.empty(8, device="cuda"), torch.empty(8, device="cuda")])
         else:
             C.op_call(C.OpKind.LayerNormBwd, [x, x, s, s], [torch.empty_like(x)])
+
+
+@pytest.mark.parametrize("n,times,cols", [(8, (1 << 21) + 1, 3), (16, (1 << 20) - 1, 5)])
+def test_rows_of_more_than_a_grid(C, n, times, cols):
+    """2^24 + 8 rows in the looping kernel (256 lanes each), and one launch's
+    rows and a few in the register kernel."""
+    R = n * times
+    r = rng(cols)
+    px = dev(r.standard_normal((n, cols)) * 2, torch.float32)
+    plab = torch.from_numpy(r.integers(0, cols, n).astype(np.int32)).cuda()
+    x, lab = repeated(px, times), repeated(plab, times)
+    x64, l64 = host(px), plab.cpu().numpy()
+    y, mx, sx = torch.zeros_like(x), torch.zeros(R, device="cuda"), torch.zeros(R, device="cuda")
+    C.op_call(C.OpKind.RowSoftmax, [x], [y, mx, sx])
+    e = np.exp(x64 - x64.max(1, keepdims=True))
+    p = e / e.sum(1, keepdims=True)
+    for got, want in ((y, p), (mx, x64.max(1)), (sx, x64.sum(1))):
+        assert orc.rel_err(host(got[:n]), want) < 1e-5 and same(got, n)
+    for op, want in ((0, x64.sum(1)), (1, x64.max(1))):
+        o = torch.zeros(R, device="cuda")
+        C.op_call(C.OpKind.RowReduce, [x], [o], RRED, struct.pack("<i", op))
+        assert orc.rel_err(host(o[:n]), want) < 1e-5 and same(o, n)
+    loss, am, rl = torch.zeros((), device="cuda"), torch.zeros(R, device="cuda", dtype=torch.int32), torch.zeros(
+        R, device="cuda")
+    C.op_call(C.OpKind.SoftmaxXent, [x, lab], [loss, y, am, rl])
+    row = np.log(e.sum(1)) + x64.max(1) - x64[np.arange(n), l64]
+    d = p.copy()
+    d[np.arange(n), l64] -= 1.0
+    assert np.array_equal(am[:n].cpu().numpy(), x64.argmax(1)) and same(am, n)
+    assert orc.rel_err(host(rl[:n]), row) < 1e-5 and same(rl, n)
+    assert orc.rel_err(host(y[:n]), d / R) < 1e-5 and same(y, n)
+    assert abs(float(loss) - row.mean()) < 1e-5 * abs(row.mean())
