@@ -297,7 +297,11 @@ Status colsum_run(const void* x, void* out, float* partial, int64_t P, int64_t M
     partial = nullptr;
   }
   const int64_t gn = (N + kNarrowLanes * VEC - 1) / (kNarrowLanes * VEC);
-  if (N >= VEC && !partial && gn <= INT32_MAX) {
+  // the vector that a ragged width moves back lies in two workgroups' columns,
+  // so a sum written over a row of x must not take that form
+  const uintptr_t xa = (uintptr_t)x, oa = (uintptr_t)out;
+  const bool apart = oa + (uintptr_t)N * (OUT_F16 ? 2 : 4) <= xa || xa + (uintptr_t)(M * N) * sizeof(TI) <= oa;
+  if (N >= VEC && (vec || apart) && !partial && gn <= INT32_MAX) {
     // one output, no partials: narrow column blocks over all rows (a
     // [8192, 4096] bf16 sum on 8 workgroups of 512 columns took 133 us).
     // At most 128 blocks (half the CUs): 1024 threads.  The f32 backward of

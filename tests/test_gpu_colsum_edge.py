@@ -31,3 +31,18 @@ def test_column_sum_edges(C, M, N, dt, offset):
     tol = 1e-5 if dout == torch.float32 else 2.0 ** -11 + 1e-5
     assert float((o.double() - ref).abs().max() / ref.abs().max()) < tol
     assert bool((of[:16] == 77).all()) and bool((of[16 + N:] == 77).all())
+
+
+@pytest.mark.parametrize("dt,M,N", [("f32", 777, 523), ("f32", 300, 9), ("f32", 500, 1001), ("f32", 300, 1024),
+                                    ("f16", 777, 517), ("f16", 300, 17), ("f16", 500, 1024)])
+@pytest.mark.parametrize("row", [0, -1])
+def test_column_sum_over_a_row_of_its_input(C, dt, M, N, row):
+    """The sums may take the place of a row: a workgroup has read its columns
+    when it writes them, and no other one reads them."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M * N)
+    x = (torch.randn((M, N), device="cuda", generator=g) + 0.25).to(DT[dt])
+    ref = x.double().sum(0)
+    C.op_call(C.OpKind.ReduceSum, [x], [x[row]])
+    tol = 1e-5 if dt == "f32" else 2.0 ** -11 + 1e-5
+    assert float((x[row].double() - ref).abs().max() / ref.abs().max()) < tol
