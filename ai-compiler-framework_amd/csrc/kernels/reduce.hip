@@ -188,9 +188,9 @@ __global__ __launch_bounds__(256) void colsum_finish_kernel(const float* __restr
 // XCD i % 8), so each line is fetched into one L2.  [8192, 4096] bf16: 16.6
 // us (4 lanes, 8 loads, no remap: 25.6 us; 1 lane: 23.3 us).
 //
-// THREADS 1024 (512 row slots) where there are few column blocks; RAG: any N
-// of at least a vector, any alignment: the last vector is moved back to end at
-// column N - 1 (columns that two lanes hold get the same bits from both).
+// THREADS 1024 (512 row slots): for few column blocks of many rows.  RAG: any
+// N of at least a vector, any alignment: the last vector is moved back to end
+// at column N - 1 (columns that two lanes hold get the same bits from both).
 constexpr int kNarrowLanes = 2;
 
 template <typename TI, bool BF16IN, bool OUT_F16, int THREADS, bool RAG>
@@ -223,13 +223,17 @@ __global__ __launch_bounds__(THREADS) void colsum_narrow_kernel(const TI* __rest
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) add_vec16<TI, BF16IN>(acc, q[u]);
     }
-    if (r < M) {  // the rest in one batch too; rows past M read the last one and add zeros
-      uint4 q[UNROLL - 1];
+    if constexpr (RAG) {
+      if (r < M) {  // the rest in one batch too; rows past M read the last one and add zeros
+        uint4 q[UNROLL - 1];
 #pragma unroll
-      for (int u = 0; u < UNROLL - 1; ++u) q[u] = get(r + u * SLOTS < M ? r + u * SLOTS : M - 1);
+        for (int u = 0; u < UNROLL - 1; ++u) q[u] = get(r + u * SLOTS < M ? r + u * SLOTS : M - 1);
 #pragma unroll
-      for (int u = 0; u < UNROLL - 1; ++u)
-        add_vec16<TI, BF16IN>(acc, r + u * SLOTS < M ? q[u] : uint4{0, 0, 0, 0});
+        for (int u = 0; u < UNROLL - 1; ++u)
+          add_vec16<TI, BF16IN>(acc, r + u * SLOTS < M ? q[u] : uint4{0, 0, 0, 0});
+      }
+    } else {
+      for (; r < M; r += SLOTS) add_vec16<TI, BF16IN>(acc, get(r));
     }
   }
 #pragma unroll
@@ -301,19 +305,29 @@ Status colsum_run(const void* x, void* out, float* partial, int64_t P, int64_t M
   // so a sum written over a row of x must not take that form
   const uintptr_t xa = (uintptr_t)x, oa = (uintptr_t)out;
   const bool apart = oa + (uintptr_t)N * (OUT_F16 ? 2 : 4) <= xa || xa + (uintptr_t)(M * N) * sizeof(TI) <= oa;
-  if (N >= VEC && (vec || apart) && !partial && gn <= INT32_MAX) {
+  // Ragged widths, against 64 scalar columns a workgroup: that kernel wins
+  // while a wave has few rows (f32 [64, 523] 1.9 us, 2.1 here; [256, 523] 3.5,
+  // 2.3; [777, 523] 8.0, 2.8) and where its N / 64 workgroups fill the chip
+  // with whole lines, which 32-byte columns at odd addresses share between
+  // XCDs (f32 [1024, 6001] 22.0, 18.0, but [384, 6001] 4.5, 7.9 and [1024,
+  // 10001] 23.0, 28.1; bf16 [1024, 10001] 22.5, 16.0, [512, 20001] 13.1, 15.6).
+  const int64_t row = N * (int64_t)sizeof(TI);
+  const bool ragged = apart && M >= 192 && (row <= (12 << 10) || (M >= 1024 && row <= (24 << 10)));
+  if (N >= VEC && (vec || ragged) && !partial && gn <= INT32_MAX) {
     // one output, no partials: narrow column blocks over all rows (a
     // [8192, 4096] bf16 sum on 8 workgroups of 512 columns took 133 us).
-    // At most 128 blocks (half the CUs): 1024 threads.  The f32 backward of
-    // 777 x 1000 x 523, whose [777, 523] sum took 9.8 us on scalar columns of
-    // 9 workgroups: 48.8 -> 39.1 us.
+    // 1024 threads: ragged on at most half the CUs from 257 rows on (the f32
+    // backward of 777 x 1000 x 523 with a [777, 523] sum: 48.8 us with the 64
+    // column kernel, 39.1), else for two blocks of 4096 rows (bf16 [16384, 16]
+    // 9.1, 6.4; more blocks gain nothing: f32 [512, 256] 2.3, 2.6, [4096, 64]
+    // 3.8, 4.0).
     const TI* xp = (const TI*)x;
 #define NARROW(T, R) colsum_narrow_kernel<TI, BF16IN, OUT_F16, T, R><<<(unsigned)gn, T, 0, s>>>(xp, out, M, N)
-    if (gn <= 128 && M > 256) {
-      if (vec) NARROW(1024, false);
-      else NARROW(1024, true);
+    if (vec) {
+      if (gn <= 2 && M >= 4096) NARROW(1024, false);
+      else NARROW(256, false);
     } else {
-      if (vec) NARROW(256, false);
+      if (gn <= 128 && M > 256) NARROW(1024, true);
       else NARROW(256, true);
     }
 #undef NARROW

@@ -46,3 +46,12 @@ def test_column_sum_over_a_row_of_its_input(C, dt, M, N, row):
     C.op_call(C.OpKind.ReduceSum, [x], [x[row]])
     tol = 1e-5 if dt == "f32" else 2.0 ** -11 + 1e-5
     assert float((x[row].double() - ref).abs().max() / ref.abs().max()) < tol
+
+
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("M,N", [(191, 33), (192, 33), (1023, 3100), (1024, 3100), (1023, 6200), (1024, 6200),
+                                 (192, 12300), (1030, 12300), (4096, 16), (4097, 8), (4095, 16)])
+def test_column_sum_around_its_rules(C, M, N, dt):
+    """The widths and row counts at which the kernel changes."""
+    for offset in (0, 1):
+        test_column_sum_edges(C, M, N, dt, offset)
