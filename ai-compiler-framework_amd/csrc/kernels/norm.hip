@@ -66,9 +66,55 @@ __device__ __forceinline__ void st_from_f32(T* p, int64_t i, float v) {
 // ===========================================================================
 // LayerNorm
 // ===========================================================================
+// Rows of at most 64 columns, one a lane, a wave per row.  In vectors such a
+// row leaves most lanes without one and pays for the masks of the last: f32
+// [4024, 49] 2.6 us against 3.0, f16 [4024, 64] without affine, backward, 2.4
+// against 3.0.
+template <typename T>
+__global__ __launch_bounds__(256) void ln_fwd_narrow_kernel(const T* x, const T* gamma, const T* beta, T* y,
+                                                            float* mean, float* rstd, int M, int N, float eps) {
+  const int c = threadIdx.x & 63;
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= M) return;  // whole wave
+  const int64_t at = (int64_t)row * N + c;
+  const float invN = 1.0f / (float)N;
+  const float v = c < N ? ld_as_f32(x, at) : 0.0f;
+  const float mu = wave_sum(v) * invN;
+  const float t = c < N ? v - mu : 0.0f;
+  const float rs = 1.0f / sqrtf(wave_sum(t * t) * invN + eps);
+  if (c < N) {
+    float o = (v - mu) * rs;
+    if (gamma) o = fmaf(o, ld_as_f32(gamma, c), ld_as_f32(beta, c));
+    st_from_f32(y, at, o);
+  }
+  if (c == 0) {
+    mean[row] = mu;
+    rstd[row] = rs;
+  }
+}
+template <typename T>
+__global__ __launch_bounds__(256) void ln_bwd_dx_narrow_kernel(const T* x, const T* dy, const T* gamma,
+                                                               const float* mean, const float* rstd, T* dx, int M,
+                                                               int N) {
+  const int c = threadIdx.x & 63;
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= M) return;
+  const int64_t at = (int64_t)row * N + c;
+  const float mu = mean[row], rs = rstd[row];
+  const float fN = (float)N, scale = rs / fN;
+  float xh = 0.0f, g = 0.0f;
+  if (c < N) {
+    xh = (ld_as_f32(x, at) - mu) * rs;
+    g = ld_as_f32(dy, at);
+    if (gamma) g *= ld_as_f32(gamma, c);
+  }
+  const float s1 = wave_sum(g), s2 = wave_sum(g * xh);
+  if (c < N) st_from_f32(dx, at, (fN * g - s1 - xh * s2) * scale);
+}
+
 // Any M and N, one wave per row (and every gridDim.x * 4 th row on), the row
-// read two or three times: rows shorter than a vector or longer than the
-// register-resident kernels hold, and more rows than one launch has lanes for.
+// read two or three times: rows longer than the register-resident kernels
+// hold, and more rows than one launch has lanes for.
 template <typename T>
 __global__ __launch_bounds__(256) void ln_fwd_loop_kernel(const T* x, const T* gamma,
                                                           const T* beta, T* y,
@@ -674,6 +720,10 @@ template <typename T>
 Status ln_fwd_run(const T* x, const T* g, const T* b, T* y, float* mean, float* rstd, int M, int N, float eps,
                   hipStream_t s) {
   const int64_t nv = ((int64_t)N + kVec<T> - 1) / kVec<T>;
+  if (N <= 64 && ln_grid_fits(M, 1)) {
+    ln_fwd_narrow_kernel<T><<<(unsigned)(((int64_t)M + 3) / 4), 256, 0, s>>>(x, g, b, y, mean, rstd, M, N, eps);
+    return launch_status("layernorm_fwd");
+  }
   if (!ln_row_fits(N, nv, kVec<T>) || !ln_grid_fits(M, nv)) {
     ln_fwd_loop_kernel<T><<<ln_loop_blocks(M), 256, 0, s>>>(x, g, b, y, mean, rstd, M, N, eps);
     return launch_status("layernorm_fwd");
@@ -735,6 +785,11 @@ Status ln_bwd_run(LnBwd<T> a, LnOut where, hipStream_t s) {
     return launch_status("layernorm_bwd");
   };
   auto dx_all = [&] {
+    if (N <= 64 && ln_grid_fits(M, 1)) {
+      ln_bwd_dx_narrow_kernel<T><<<(unsigned)(((int64_t)M + 3) / 4), 256, 0, s>>>(a.x, a.dy, a.gamma, a.mean, a.rstd,
+                                                                                  a.dx, M, N);
+      return launch_status("layernorm_bwd");
+    }
     if (fits) return rows(M, 0, false);
     ln_bwd_dx_loop_kernel<T><<<ln_loop_blocks(M), 256, 0, s>>>(a.x, a.dy, a.gamma, a.mean, a.rstd, a.dx, M, N);
     return launch_status("layernorm_bwd");
