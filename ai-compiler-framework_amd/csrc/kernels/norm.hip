@@ -112,37 +112,36 @@ __global__ __launch_bounds__(256) void ln_bwd_dx_narrow_kernel(const T* x, const
   if (c < N) st_from_f32(dx, at, (fN * g - s1 - xh * s2) * scale);
 }
 
-// Any M and N, one wave per row (and every gridDim.x * 4 th row on), the row
-// read two or three times: rows longer than the register-resident kernels
-// hold, and more rows than one launch has lanes for.
+// Any N, one wave per row, the row read two or three times: rows longer than
+// the register-resident kernels hold.
 template <typename T>
 __global__ __launch_bounds__(256) void ln_fwd_loop_kernel(const T* x, const T* gamma,
                                                           const T* beta, T* y,
                                                           float* mean, float* rstd,
                                                           int M, int N, float eps) {
   const int lane = threadIdx.x & 63;
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= M) return;  // whole wave
+  const T* xr = x + (int64_t)row * N;
+  T* yr = y + (int64_t)row * N;
   const float invN = 1.0f / (float)N;
-  for (int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); row < M; row += (int64_t)gridDim.x * 4) {
-    const T* xr = x + row * N;
-    T* yr = y + row * N;
-    float s = 0.0f;
-    for (int c = lane; c < N; c += 64) s += ld_as_f32(xr, c);
-    const float mu = wave_sum(s) * invN;
-    float d = 0.0f;
-    for (int c = lane; c < N; c += 64) {
-      const float t = ld_as_f32(xr, c) - mu;
-      d = fmaf(t, t, d);
-    }
-    const float rs = 1.0f / sqrtf(wave_sum(d) * invN + eps);
-    for (int c = lane; c < N; c += 64) {
-      float o = (ld_as_f32(xr, c) - mu) * rs;
-      if (gamma) o = fmaf(o, ld_as_f32(gamma, c), ld_as_f32(beta, c));
-      st_from_f32(yr, c, o);
-    }
-    if (lane == 0) {
-      mean[row] = mu;
-      rstd[row] = rs;
-    }
+  float s = 0.0f;
+  for (int c = lane; c < N; c += 64) s += ld_as_f32(xr, c);
+  const float mu = wave_sum(s) * invN;
+  float d = 0.0f;
+  for (int c = lane; c < N; c += 64) {
+    const float t = ld_as_f32(xr, c) - mu;
+    d = fmaf(t, t, d);
+  }
+  const float rs = 1.0f / sqrtf(wave_sum(d) * invN + eps);
+  for (int c = lane; c < N; c += 64) {
+    float o = (ld_as_f32(xr, c) - mu) * rs;
+    if (gamma) o = fmaf(o, ld_as_f32(gamma, c), ld_as_f32(beta, c));
+    st_from_f32(yr, c, o);
+  }
+  if (lane == 0) {
+    mean[row] = mu;
+    rstd[row] = rs;
   }
 }
 
@@ -155,29 +154,28 @@ __global__ __launch_bounds__(256) void ln_bwd_dx_loop_kernel(const T* x, const T
                                                              const float* rstd, T* dx,
                                                              int M, int N) {
   const int lane = threadIdx.x & 63;
-  const float fN = (float)N;
-  for (int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); row < M; row += (int64_t)gridDim.x * 4) {
-    const T* xr = x + row * N;
-    const T* dyr = dy + row * N;
-    T* dxr = dx + row * N;
-    const float mu = mean[row], rs = rstd[row];
-    const float scale = rs / fN;
-    float s1 = 0.0f, s2 = 0.0f;
-    for (int c = lane; c < N; c += 64) {
-      const float xh = (ld_as_f32(xr, c) - mu) * rs;
-      float g = ld_as_f32(dyr, c);
-      if (gamma) g *= ld_as_f32(gamma, c);
-      s1 += g;
-      s2 = fmaf(g, xh, s2);
-    }
-    s1 = wave_sum(s1);
-    s2 = wave_sum(s2);
-    for (int c = lane; c < N; c += 64) {
-      const float xh = (ld_as_f32(xr, c) - mu) * rs;
-      float g = ld_as_f32(dyr, c);
-      if (gamma) g *= ld_as_f32(gamma, c);
-      st_from_f32(dxr, c, (fN * g - s1 - xh * s2) * scale);
-    }
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= M) return;
+  const T* xr = x + (int64_t)row * N;
+  const T* dyr = dy + (int64_t)row * N;
+  T* dxr = dx + (int64_t)row * N;
+  const float mu = mean[row], rs = rstd[row];
+  const float fN = (float)N, scale = rs / fN;
+  float s1 = 0.0f, s2 = 0.0f;
+  for (int c = lane; c < N; c += 64) {
+    const float xh = (ld_as_f32(xr, c) - mu) * rs;
+    float g = ld_as_f32(dyr, c);
+    if (gamma) g *= ld_as_f32(gamma, c);
+    s1 += g;
+    s2 = fmaf(g, xh, s2);
+  }
+  s1 = wave_sum(s1);
+  s2 = wave_sum(s2);
+  for (int c = lane; c < N; c += 64) {
+    const float xh = (ld_as_f32(xr, c) - mu) * rs;
+    float g = ld_as_f32(dyr, c);
+    if (gamma) g *= ld_as_f32(gamma, c);
+    st_from_f32(dxr, c, (fN * g - s1 - xh * s2) * scale);
   }
 }
 
@@ -705,35 +703,45 @@ bool ln_bwd_check(const TensorDesc* in, int ni, const TensorDesc* out, int no, D
   else CALL(1024, 4)
 constexpr int kLnMaxVecs = 4096;  // longer rows take the looping kernels
 
-// Whether rows of nv vectors fit the register-resident kernels, and whether M
-// of them fit one launch: the runtime counts a grid's lanes in 32 bits and
-// starts too few workgroups, without an error, above that.
-constexpr bool ln_row_fits(int64_t N, int64_t nv, int V) { return N >= V && nv <= kLnMaxVecs; }
-constexpr bool ln_grid_fits(int64_t M, int64_t nv) {
+// Rows of nv vectors that one launch takes: the runtime counts a grid's lanes
+// in 32 bits and starts too few workgroups, without an error, above that.
+constexpr int64_t ln_rows_per_launch(int64_t nv) {
   int64_t lanes = 64;
-  while (nv > 4 * lanes) lanes *= 2;
-  return M * lanes <= (int64_t)UINT32_MAX - 1024;
+  while (lanes < 1024 && nv > 4 * lanes) lanes *= 2;
+  return ((int64_t)UINT32_MAX - 1024) / lanes;
 }
-unsigned ln_loop_blocks(int64_t M) { return (unsigned)((M + 3) / 4 < 1 << 22 ? (M + 3) / 4 : 1 << 22); }
+// launch(first row, rows) for every part of M rows.  No rows: one launch, of an
+// empty grid, which refuses the call.
+template <typename F>
+Status ln_row_parts(int64_t M, int64_t nv, F&& launch) {
+  const int64_t most = ln_rows_per_launch(nv);
+  int64_t r = 0;
+  do {
+    const Status st = launch(r, (int)(M - r < most ? M - r : most));
+    if (st != Status::Ok) return st;
+    r += most;
+  } while (r < M);
+  return Status::Ok;
+}
 
 template <typename T>
-Status ln_fwd_run(const T* x, const T* g, const T* b, T* y, float* mean, float* rstd, int M, int N, float eps,
-                  hipStream_t s) {
+Status ln_fwd_run(const T* x0, const T* g, const T* b, T* y0, float* mean0, float* rstd0, int64_t all, int N,
+                  float eps, hipStream_t s) {
   const int64_t nv = ((int64_t)N + kVec<T> - 1) / kVec<T>;
-  if (N <= 64 && ln_grid_fits(M, 1)) {
-    ln_fwd_narrow_kernel<T><<<(unsigned)(((int64_t)M + 3) / 4), 256, 0, s>>>(x, g, b, y, mean, rstd, M, N, eps);
-    return launch_status("layernorm_fwd");
-  }
-  if (!ln_row_fits(N, nv, kVec<T>) || !ln_grid_fits(M, nv)) {
-    ln_fwd_loop_kernel<T><<<ln_loop_blocks(M), 256, 0, s>>>(x, g, b, y, mean, rstd, M, N, eps);
-    return launch_status("layernorm_fwd");
-  }
+  return ln_row_parts(all, nv, [&](int64_t r, int M) {
+    const T* x = x0 + r * N;
+    T* y = y0 + r * N;
+    float *mean = mean0 + r, *rstd = rstd0 + r;
 #define LN_FWD(LPR, VPT)                                                                                   \
   ln_fwd_kernel<T, LPR, VPT><<<(unsigned)(((int64_t)M * LPR + ln_threads(LPR) - 1) / ln_threads(LPR)),    \
                                ln_threads(LPR), 0, s>>>(x, g, b, y, mean, rstd, M, N, eps)
-  LN_BY_WIDTH(LN_FWD);
+    const unsigned by_wave = (unsigned)(((int64_t)M + 3) / 4);
+    if (N <= 64) ln_fwd_narrow_kernel<T><<<by_wave, 256, 0, s>>>(x, g, b, y, mean, rstd, M, N, eps);
+    else if (nv > kLnMaxVecs) ln_fwd_loop_kernel<T><<<by_wave, 256, 0, s>>>(x, g, b, y, mean, rstd, M, N, eps);
+    else LN_BY_WIDTH(LN_FWD);
 #undef LN_FWD
-  return launch_status("layernorm_fwd");
+    return launch_status("layernorm_fwd");
+  });
 }
 
 // Whether out[k] shares no byte with an input or another output.
@@ -763,7 +771,6 @@ Status ln_bwd_run(LnBwd<T> a, LnOut where, hipStream_t s) {
   const int M = a.M, N = a.N;
   const int64_t nv = ((int64_t)N + V - 1) / V;
   const bool affine = a.dgamma != nullptr;
-  const bool regs = ln_row_fits(N, nv, V), fits = regs && ln_grid_fits(M, nv);
   auto sums_loop = [&] {
     ln_bwd_dgdb_loop_kernel<T><<<(unsigned)(((int64_t)N + 63) / 64), 256, 0, s>>>(a.x, a.dy, a.mean, a.rstd,
                                                                                 a.dgamma, a.dbeta, M, N);
@@ -774,7 +781,7 @@ Status ln_bwd_run(LnBwd<T> a, LnOut where, hipStream_t s) {
     return st == Status::Ok ? second() : st;
   };
   const unsigned col_blocks = (unsigned)((nv + kLnColLanes - 1) / kLnColLanes);
-  auto rows = [&](int64_t n, unsigned extra, bool reserved) {
+  auto rows = [&](const LnBwd<T>& a, int64_t n, unsigned extra, bool reserved) {
 #define LN_BWD(LPR, VPT)                                                                                 \
   do {                                                                                                   \
     const unsigned rb = (unsigned)((n * LPR + ln_threads(LPR) - 1) / ln_threads(LPR));                   \
@@ -785,21 +792,29 @@ Status ln_bwd_run(LnBwd<T> a, LnOut where, hipStream_t s) {
     return launch_status("layernorm_bwd");
   };
   auto dx_all = [&] {
-    if (N <= 64 && ln_grid_fits(M, 1)) {
-      ln_bwd_dx_narrow_kernel<T><<<(unsigned)(((int64_t)M + 3) / 4), 256, 0, s>>>(a.x, a.dy, a.gamma, a.mean, a.rstd,
-                                                                                  a.dx, M, N);
+    return ln_row_parts(M, nv, [&](int64_t r, int n) {
+      LnBwd<T> p = a;
+      p.x += r * N;
+      p.dy += r * N;
+      p.dx += r * N;
+      p.mean += r;
+      p.rstd += r;
+      p.M = n;
+      if (N > 64 && nv <= kLnMaxVecs) return rows(p, n, 0, false);
+      const unsigned by_wave = (unsigned)(((int64_t)n + 3) / 4);
+      if (N <= 64)
+        ln_bwd_dx_narrow_kernel<T><<<by_wave, 256, 0, s>>>(p.x, p.dy, p.gamma, p.mean, p.rstd, p.dx, n, N);
+      else
+        ln_bwd_dx_loop_kernel<T><<<by_wave, 256, 0, s>>>(p.x, p.dy, p.gamma, p.mean, p.rstd, p.dx, n, N);
       return launch_status("layernorm_bwd");
-    }
-    if (fits) return rows(M, 0, false);
-    ln_bwd_dx_loop_kernel<T><<<ln_loop_blocks(M), 256, 0, s>>>(a.x, a.dy, a.gamma, a.mean, a.rstd, a.dx, M, N);
-    return launch_status("layernorm_bwd");
+    });
   };
-  if (!affine || M < 1) return dx_all();  // no rows: refused as an empty grid
+  if (!affine || M < 1) return dx_all();
   // dx, then the sums, 64 columns a workgroup (which has read all of them when
   // it writes): the sums may lie on gamma, and at N <= 64 on any input
   if (where == LnOut::OnSums) return in_order(dx_all, sums_loop);
   // the kernels below step 32-bit row indices to less than 1024 past M
-  if (!regs || M > INT32_MAX - 1024) return in_order(sums_loop, dx_all);
+  if (N < V || nv > kLnMaxVecs || M > INT32_MAX - 1024) return in_order(sums_loop, dx_all);
   // Large matrices: x and dy read once, P chunks of rows (one workgroup per
   // CU), partial sums in dx.  Below 16 MiB (x and dy together an eighth of the
   // 256 MB MALL) the second read of the one-launch form comes from the caches
@@ -827,16 +842,16 @@ Status ln_bwd_run(LnBwd<T> a, LnOut where, hipStream_t s) {
     ln_bwd_finish_kernel<T><<<(unsigned)((2 * (int64_t)N + 63) / 64), 1024, 0, s>>>(a);
     st = launch_status("layernorm_bwd_finish");
     if (st != Status::Ok) return st;
-    return rows((int64_t)a.P * a.RS, 0, true);
+    return rows(a, (int64_t)a.P * a.RS, 0, true);
   }
-  if (where == LnOut::OnDx || nv > 2048 || !fits) {  // two launches: the sums before dx, or its rows take other workgroups
+  if (where == LnOut::OnDx || nv > 2048) {  // two launches: the sums before dx, or its rows take wider workgroups
     auto columns = [&] {
       ln_bwd_columns_kernel<T><<<col_blocks, kLnColThreads, 0, s>>>(a);
       return launch_status("layernorm_bwd_columns");
     };
     return in_order(columns, dx_all);
   }
-  return rows(M, col_blocks, false);
+  return rows(a, M, col_blocks, false);
 }
 
 #define LN_VARIANTS(SFX, T, D)                                                                          \
