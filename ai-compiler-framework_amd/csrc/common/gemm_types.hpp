@@ -48,7 +48,34 @@ struct GemmParams {
   int tiles_m, tiles_n;
   GemmAdamW adam;  // ACT_ADAMW only
   float* colsum;   // ACT_DGELU, bf16 out: per-tile column sums of C, row m0/256 of [M/256, N]
+  int apart;       // set by run_gemm: gemm_outputs_apart
 };
+
+// Whether no byte that the call writes (es, os: bytes of an operand's and an
+// output's element) lies in A or B.  A product written over an operand is
+// right where one tile spans N (over A) or M (over B): its workgroup has read
+// all that it overwrites, and no other one reads it.  Such a call keeps to the
+// largest exact tiles, and to the general-stride kernel where none fits; tiles
+// that read their neighbours' rows and smaller ones would break it.
+inline bool gemm_outputs_apart(const GemmParams& p, int64_t es, int64_t os) {
+  struct Range {
+    uintptr_t lo, hi;
+  };
+  auto range = [](const void* d, int64_t r, int64_t rs, int64_t c, int64_t cs, int64_t size) {
+    const uintptr_t lo = reinterpret_cast<uintptr_t>(d);
+    return Range{lo, lo + (uintptr_t)(((r - 1) * rs + (c - 1) * cs + 1) * size)};
+  };
+  const Range in[2] = {range(p.A, p.M, p.a_rs, p.K, p.a_cs, es), range(p.B, p.K, p.b_rs, p.N, p.b_cs, es)};
+  auto apart = [&](const void* d, int64_t ld, int64_t cs, int64_t size) {
+    const Range o = range(d, p.M, ld, p.N, cs, size);
+    return !d || ((o.hi <= in[0].lo || in[0].hi <= o.lo) && (o.hi <= in[1].lo || in[1].hi <= o.lo));
+  };
+  if (!apart(p.C, p.c_rs, p.c_cs, os)) return false;
+  if (p.act == ACT_GELU && !apart(p.aux, p.aux_rs, 1, os)) return false;
+  if (p.act == ACT_ADAMW)
+    return apart(p.adam.M, p.c_rs, 1, 4) && apart(p.adam.V, p.c_rs, 1, 4) && apart(p.adam.Wb, p.c_rs, 1, 2);
+  return true;
+}
 
 template <int IN>
 struct InTraits;

@@ -1383,7 +1383,7 @@ Status run_nt256(const GemmParams& g, hipStream_t s) {
 // aligned bases and rows; C (and the aux matrix) have unit column stride with
 // 16-byte aligned rows, and bias is contiguous.  K is whole K-steps, and the
 // shape tiles exactly or, where the output is only written (no update in
-// place, no column sums, no pre-activation read from the output's memory),
+// place, no column sums, no operand or pre-activation in the output's memory),
 // the last tiles are moved back to end at M and N: columns, and rows of an
 // M-contiguous A, then have to be whole 16-byte chunks, and the tiles may hold
 // a quarter more than the output (above that the next smaller tile or the edge
@@ -1403,7 +1403,7 @@ bool nt_eligible(const GemmParams& p, int BM, int BN, bool mn_ok) {
   if (p.K % (128 / ES)) return false;
   if (p.M % BM || p.N % BN) {
     constexpr int64_t CE = 16 / ES, CO = OUT == OUT_F32 ? 4 : 8;
-    if (p.act == ACT_ADAMW || p.colsum || p.M < BM || p.N < BN) return false;
+    if (p.act == ACT_ADAMW || p.colsum || !p.apart || p.M < BM || p.N < BN) return false;
     if (p.M % BM && p.a_mode != LD_KCONTIG && p.M % CE) return false;
     if (p.N % BN && (p.N % CO || (p.b_mode != LD_KCONTIG && p.N % CE))) return false;
     const int64_t rows = (p.M + BM - 1) / BM * BM, cols = (p.N + BN - 1) / BN * BN;
@@ -1459,12 +1459,13 @@ __global__ __launch_bounds__(512) void tile_colsum_kernel(const uint16_t* __rest
 
 template <int IN, int OUT>
 Status run_gemm(GemmParams& p, hipStream_t s) {
+  p.apart = gemm_outputs_apart(p, IN == IN_F32 ? 4 : 2, OUT == OUT_F32 ? 4 : 2);
   if (p.colsum) {  // dGELU with column sums, bf16 output, M and N multiples of 256
     if constexpr (OUT == OUT_BF16 && IN != IN_F32) {
       if (p.act == ACT_DGELU && nt_eligible<IN, OUT>(p, 256, 256, true)) {
         // the column sums live in the 8-wave 256 x 256 configuration's
         // epilogue (whole tile in one pass): dispatch to it directly
-        if ((p.M / 256) * (p.N / 256) >= 128) return run_nt<IN, OUT, 256, 256, 2, 4, true>(p, s);
+        if ((p.M / 256) * (p.N / 256) >= 128 || !p.apart) return run_nt<IN, OUT, 256, 256, 2, 4, true>(p, s);
         // fewer of those tiles than half the CUs: smaller ones, then the sums
         // from the stored output, in the same order (256 x 3584 x 3584: 72 ->
         // 21 us, 2048^3 49 -> 28; same bits)
@@ -1489,7 +1490,7 @@ Status run_gemm(GemmParams& p, hipStream_t s) {
         // -> 85, 2560 x 2560 x 4096 122 -> 87 (400 tiles of 128 x 128)
         const int64_t tiles128 = (p.M / 128) * (p.N / 128);
         const bool deep = p.K >= 16 * 64;
-        if (tiles128 >= 512) return run_nt256<IN, OUT>(p, s);
+        if (tiles128 >= 512 || !p.apart) return run_nt256<IN, OUT>(p, s);
         if (tiles128 >= 128) {
           if (deep && tiles128 <= 256) return run_nt<IN, OUT, 128, 128, 2, 2, true, 4>(p, s);
           return run_nt<IN, OUT, 128, 128, 2, 2, true>(p, s);
@@ -1575,7 +1576,7 @@ Status run_gemm(GemmParams& p, hipStream_t s) {
     // (fp32 is bound by its MFMAs, so by the tiles of the fullest CU: 2048 x
     // 1024 x 512 33.4 us on 128 CUs with a 128 x 128 tile each, 18.9 on 64 x 64;
     // 4096 x 512 x 1024 62.5, 33.5)
-    if (tiles128 >= (IN == IN_F32 ? 384 : 128) && nt_eligible<IN, OUT>(p, 128, 128, true)) {
+    if (tiles128 >= (IN == IN_F32 && p.apart ? 384 : 128) && nt_eligible<IN, OUT>(p, 128, 128, true)) {
       if constexpr (IN != IN_F32) {
         if (deep && tiles128 <= 256) return run_nt<IN, OUT, 128, 128, 2, 2, true, 4>(p, s);
       }

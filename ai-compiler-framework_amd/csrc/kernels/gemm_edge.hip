@@ -512,7 +512,7 @@ Status run_edge_tiles(const GemmParams& g, hipStream_t s) {
 
 bool edge_gemm_ok(const GemmParams& p, int in) {
   const int64_t es = in == IN_F32 ? 4 : 2, ce = 16 / es;
-  if (p.colsum || p.act == ACT_ADAMW || p.c_cs != 1) return false;
+  if (p.colsum || p.act == ACT_ADAMW || p.c_cs != 1 || !p.apart) return false;
   if (p.M > INT32_MAX / 2 || p.N > INT32_MAX / 2 || p.K > INT32_MAX / 2 || p.K < ce) return false;
   // 32-bit offsets from a tile's first row, for the up to 256 rows of it
   auto operand_ok = [&](int mode, int64_t ld_k, int64_t ld_mn, int64_t mn) {
