@@ -1586,10 +1586,16 @@ Status run_gemm(GemmParams& p, hipStream_t s) {
     // 112.6 -> 19.8 us, fp32 1024^3 NN 53.8 -> 19.7 us against the
     // general-stride kernel)
     constexpr bool MN64 = true;
-    // (fp32 is bound by its MFMAs, so by the tiles of the fullest CU: 2048 x
-    // 1024 x 512 33.4 us on 128 CUs with a 128 x 128 tile each, 18.9 on 64 x 64;
-    // 4096 x 512 x 1024 62.5, 33.5)
-    if (tiles128 >= (IN == IN_F32 && p.apart ? 384 : 128) && nt_eligible<IN, OUT>(p, 128, 128, true)) {
+    // fp32 is bound by its MFMAs, so by the work of the fullest CU, counted here
+    // in 64 x 64 tiles: 2048 x 1024 x 512 takes 33.5 us as one 128 x 128 tile on
+    // each of 128 CUs, 17.9 as two 64 x 64 tiles each; 2048 x 2176 x 2048 233,
+    // 151.  Where both load it alike, short K gains from the finer tiles (2048 x
+    // 1792 x 128 12.1, 11.0), long K from reading half the operand bytes (2048 x
+    // 2048 x 4096 NT 236, 254).  From 384 tiles of 128 x 128 on, 128 x 128.
+    const int64_t round64 = (((p.M + 63) / 64) * ((p.N + 63) / 64) + 255) / 256, round128 = 4 * ((tiles128 + 255) / 256);
+    const bool smaller = IN == IN_F32 && p.apart && tiles128 < 384 &&
+                         (round64 < round128 || (round64 == round128 && p.K <= 512));
+    if (tiles128 >= 128 && !smaller && nt_eligible<IN, OUT>(p, 128, 128, true)) {
       if constexpr (IN != IN_F32) {
         if (deep && tiles128 <= 256) return run_nt<IN, OUT, 128, 128, 2, 2, true, 4>(p, s);
       }

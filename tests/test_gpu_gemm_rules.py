@@ -45,3 +45,9 @@ def check(C, M, N, K, dt, kinds=()):
 def test_shapes_of_whole_smaller_tiles(C, M, N, K, dt):
     """Multiples of 64 and of 128 that larger tiles would have to move back."""
     check(C, M, N, K, dt, (3, 5) if dt != "bf16_f32" else ())
+
+
+@pytest.mark.parametrize("M,N,K", [(2048, 1536, 1024), (2048, 1792, 512), (2048, 1792, 544), (2048, 2048, 512),
+                                   (2048, 2048, 1056), (2048, 2176, 1024), (3072, 2048, 128)])
+def test_fp32_tiles_by_the_fullest_cu(C, M, N, K):
+    check(C, M, N, K, "f32")
