@@ -1518,12 +1518,17 @@ Status run_gemm(GemmParams& p, hipStream_t s) {
     // fewer than 128 tiles of 64 x 64: one 16 x 16 tile per wave with K split
     // over the waves of a workgroup reaches more CUs than any tiled
     // configuration, and reads every operand layout in place.  Above 512
-    // such tiles (two workgroups a CU) it re-reads the operands from L2 too
-    // often: 512^3 11.2 us against 7.1 on the edge kernel's K-split tiles,
-    // 300 x 1001 x 2000 50 against 30, but 300 x 300 x 1000 9.3 against 11.0.
+    // such tiles (two workgroups a CU) it re-reads the operands from L2 often
+    // and long K goes to the edge kernel's K-split tiles: 512 x 512 x 1024 NN
+    // 15.8 us, 10.1 there, NT 20.2, 9.4; 300 x 1001 x 2000 NN 45.7, 31.5.  Short
+    // K stays, with whole 16 x 16 tiles to K = 511 (512 x 512 x 384 NN 6.5, 8.2;
+    // NT 8.0, 8.3), else to 319 (1000 x 200 x 256 NN 5.1, 5.3, NT 6.2, 5.2, x 384
+    // 6.6, 6.2; 4096 x 60 x 384 TN 14.4, 6.3), and to 255 from 1408 tiles on (768
+    // x 512 x 256 NN 6.7, 6.4, NT 8.0, 6.4).
     const int64_t tiles64 = ((p.M + 63) / 64) * ((p.N + 63) / 64);
     const int64_t tiles16 = ((p.M + 15) / 16) * ((p.N + 15) / 16);
-    const bool split = tiles16 > 512 && p.K >= 256 && edge_gemm_ok(p, IN);
+    const bool whole = p.M % 16 == 0 && p.N % 16 == 0 && p.N >= 64;
+    const bool split = tiles16 > 512 && p.K >= (tiles16 >= 1408 ? 256 : whole ? 512 : 320) && edge_gemm_ok(p, IN);
     if (tiles64 < kSmallGemmMaxTiles64 && !split && (p.act == ACT_NONE || p.act == ACT_RELU) && p.c_cs == 1 && !p.aux) {
       SmallGemm g{};
       g.A = (const float*)p.A;

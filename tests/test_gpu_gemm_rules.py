@@ -51,3 +51,9 @@ def test_shapes_of_whole_smaller_tiles(C, M, N, K, dt):
                                    (2048, 2048, 1056), (2048, 2176, 1024), (3072, 2048, 128)])
 def test_fp32_tiles_by_the_fullest_cu(C, M, N, K):
     check(C, M, N, K, "f32")
+
+
+@pytest.mark.parametrize("M,N,K", [(512, 512, 508), (512, 512, 512), (1024, 256, 256), (528, 512, 320), (1000, 200, 319),
+                                   (1000, 200, 320), (688, 512, 256), (704, 512, 256), (8000, 32, 320)])
+def test_fp32_few_tiles(C, M, N, K):
+    check(C, M, N, K, "f32")
