@@ -1737,17 +1737,16 @@ bool epi_check(const TensorDesc* in, int ni, const TensorDesc* out, int no, cons
         W.shape[0] < C.rows / 256)
       return false;
     if (!fin && W.shape[0] != C.rows / 256) return false;  // its reader sums every row
-    // the column sums are kept per 256-row block: accept exactly the calls
+    // the column sums are kept per 256-row block: accept exactly the shapes
     // that run_gemm takes with them (M, N multiples of 256, so the workspace
-    // has at least one row; K of 64; aligned operands)
-    if (din != DType::kBF16) return false;
+    // has at least one row; K of 64; aligned operands), also of a descriptor
+    // whose workspace has no memory yet
+    if (din != DType::kBF16 || C.rows % 256 || C.cols % 256) return false;
     GemmParams p{};
     fill_operands(p, in[0], in[1], out[0], e.ta, e.tb);
     p.act = ACT_DGELU;
     p.aux = const_cast<void*>(X.data);
     p.aux_rs = X.stride[0];
-    p.colsum = (float*)W.data;
-    if (!p.colsum) return false;
     return nt_eligible<IN_BF16, OUT_BF16>(p, 256, 256, true);
   }
   if (no > 2) return false;
@@ -1805,6 +1804,7 @@ Status epi_launch_common(const TensorDesc* in, int no, TensorDesc* out, const vo
     return dispatch_gemm(p, din, dout, as_stream(stream));
   }
   if (e.kind == AICF_EPI_DGELU_COLSUM) {
+    if (!out[2].data) return Status::InvalidArgument;
     p.colsum = (float*)out[2].data;
     const Status st = dispatch_gemm(p, din, dout, as_stream(stream));
     if (st != Status::Ok) return st;

@@ -243,6 +243,17 @@ def test_dgelu_colsum_supported_only_where_it_runs(lib):
     assert _call(lib, 17, ins, outs, gepi, pay) == NOTIMPL
 
 
+def test_dgelu_colsum_of_a_descriptor_without_memory(lib):
+    """Support is a matter of shapes, types and alignment: a workspace that has
+    no memory yet is supported, and its launch refused on the host."""
+    gepi = int.from_bytes(b"GEPI", "little")
+    ins = [d((512, 64), BF16, FAKE), d((64, 256), BF16, FAKE + (1 << 24)), d((512, 256), BF16, FAKE + (2 << 24))]
+    outs = [d((512, 256), BF16, FAKE + (3 << 24)), d((256,), F32, FAKE + (4 << 24)), d((2, 256), F32, None)]
+    assert _call(lib, 17, ins, outs, gepi, struct.pack("<iii", 0, 0, 6)) == INV  # unsupported: NotImplemented
+    outs[0] = d((512, 256), BF16, FAKE + 8 + (3 << 24))
+    assert _call(lib, 17, ins, outs, gepi, struct.pack("<iii", 0, 0, 6)) == NOTIMPL
+
+
 def test_zero_size_inputs_follow_the_reference(lib):
     """Zero-element tensors get the reference's statuses, decided on the host:
     copy, grad_zero and Adam accept n = 0 and return Ok without a launch
