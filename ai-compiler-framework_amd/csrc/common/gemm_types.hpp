@@ -200,6 +200,13 @@ __device__ __forceinline__ int nt_mn_swizzle(int k) {
 // gemm_edge.hip: C = epi(op(A) . op(B)) for any M, N, K >= 16 bytes and any
 // alignment, operands K- or M/N-contiguous, C with unit column stride.
 bool edge_gemm_ok(const GemmParams& p, int in);
+// Whether a 16-bit product of whole smaller tiles runs there all the same: at
+// most one 32 x 32 tile a CU and long K, which eight groups of waves share
+// (64 x 256 x 4096 11.6 -> 9.7 us, 256 x 1024 x 4096 12.0 -> 10.5 against the
+// 64 x 64 tiles with 8 stages; M-contiguous A from K = 4096: 256 x 256 x 8192
+// 23.1 -> 17.5, 512 x 512 x 4096 equal).  Plain and AdamW products alike: an
+// update has the same bits with and without the separate gradient.
+bool edge_splits_k(const GemmParams& p, int in);
 Status edge_gemm(GemmParams& p, int in, int out, void* stream);
 
 }  // namespace aicf::hip

@@ -1498,9 +1498,11 @@ Status run_gemm(GemmParams& p, hipStream_t s) {
     if constexpr (OUT == OUT_F32 && IN == IN_BF16) {
       if (nt_eligible<IN, OUT>(p, 256, 256, true)) {
         // the largest tiles that give every other CU one, as for the other
-        // epilogues (the gradient's bits are the same: K order does not depend
-        // on the tile): 1024 x 1024 x 8192 174 -> 37 us, 2048 x 2048 x 8192 181
-        // -> 85, 2560 x 2560 x 4096 122 -> 87 (400 tiles of 128 x 128)
+        // epilogues: 1024 x 1024 x 8192 174 -> 37 us, 2048 x 2048 x 8192 181 ->
+        // 85, 2560 x 2560 x 4096 122 -> 87 (400 tiles of 128 x 128).  The
+        // gradient has the plain product's bits: K order does not depend on the
+        // tile, and K is split where the plain product splits it.
+        if (edge_splits_k(p, IN)) return edge_gemm(p, IN, OUT, s);
         const int64_t tiles128 = (p.M / 128) * (p.N / 128);
         const bool deep = p.K >= 16 * 64;
         if (tiles128 >= 512 || !p.apart) return run_nt256<IN, OUT>(p, s);
@@ -1606,14 +1608,8 @@ Status run_gemm(GemmParams& p, hipStream_t s) {
       }
       return run_nt<IN, OUT, 128, 128, 2, 2, true>(p, s);
     }
-    // at most one 32 x 32 tile a CU and K >= 2048: the edge kernel splits K
-    // eight ways (64 x 256 x 4096 11.6 -> 9.7 us, 256 x 1024 x 4096 12.0 ->
-    // 10.5 against the 64 x 64 tiles with 8 stages; M-contiguous A from K =
-    // 4096: 256 x 256 x 8192 23.1 -> 17.5, 512 x 512 x 4096 equal)
     if constexpr (IN != IN_F32) {
-      const int64_t tiles32 = ((p.M + 31) / 32) * ((p.N + 31) / 32);
-      if (tiles32 <= 256 && p.K >= (p.a_mode == LD_KCONTIG ? 2048 : 4096) && edge_gemm_ok(p, IN))
-        return edge_gemm(p, IN, OUT, s);
+      if (edge_splits_k(p, IN)) return edge_gemm(p, IN, OUT, s);
     }
     // fewer tiles than CUs at 128x128: 64x64 tiles (4 waves of 32x32)
     if (nt_eligible<IN, OUT>(p, 64, 64, MN64)) {

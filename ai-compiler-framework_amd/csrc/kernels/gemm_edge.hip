@@ -1,7 +1,8 @@
 // GEMM on MFMA for sizes that no exact tiling covers: any M, N and K, any
 // element alignment, operands K-contiguous ([MN][K] in memory) or
 // M/N-contiguous ([K][MN]), every epilogue of gemm.hip except the column sums
-// and the fused AdamW.
+// (AdamW on whole tiles with K split, for the weights that a plain product
+// would compute there).
 //
 //   C[M,N] = epi( op(A)[M,K] . op(B)[K,N] )
 //
@@ -40,6 +41,7 @@ struct EdgeParams {
   int M, N, K;
   int bias_f32, act;
   int tiles_m, tiles_n;
+  GemmAdamW adam;  // ADAM only
 };
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -177,7 +179,9 @@ struct EdgeOperand {
   }
 };
 
-template <int IN, int OUT, int BM, int BN, int WM, int WN, int KSPL, int PD, bool AKC, bool BKC>
+// ADAM: the tile is the gradient of a weight matrix; AdamW is applied to it
+// instead of storing it (whole tiles, 16-byte aligned rows).
+template <int IN, int OUT, int BM, int BN, int WM, int WN, int KSPL, int PD, bool AKC, bool BKC, bool ADAM>
 __global__ __launch_bounds__(64 * WM * WN * KSPL) void gemm_edge_kernel(EdgeParams p) {
   constexpr int ES = IN == IN_F32 ? 4 : 2;
   constexpr int MS = ES == 2 ? 16 : 32;             // 16 x 16 x 32, or fp32 32 x 32 x 2
@@ -383,6 +387,34 @@ __global__ __launch_bounds__(64 * WM * WN * KSPL) void gemm_edge_kernel(EdgePara
   // Epilogue from the registers: lane (fr, fh) holds 4 consecutive columns of
   // one row per accumulator quad.
   constexpr int G = MS == 32 ? 4 : 1;
+  if constexpr (ADAM) {
+    static_assert(G == 1 && OUT == OUT_F32, "bf16 operands, fp32 gradient");
+    const AdamWScalars sc = adamw_scalars(p.adam.step, p.adam.args);
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) {
+        const int64_t e = (m0 + wm * WTM + j * MS + fr) * p.ldc + n0 + wn * WTN + i * MS + 4 * fh;
+        f32x4 pp = *reinterpret_cast<const f32x4*>(p.adam.P + e);
+        f32x4 mm = *reinterpret_cast<const f32x4*>(p.adam.M + e);
+        f32x4 vv = *reinterpret_cast<const f32x4*>(p.adam.V + e);
+        u16x4 w;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          float pk = pp[k], mk = mm[k], vk = vv[k];
+          adamw_elem(pk, acc[i][j][k], mk, vk, sc, p.adam.args);
+          pp[k] = pk;
+          mm[k] = mk;
+          vv[k] = vk;
+          w[k] = f32_to_bf16(pk);
+        }
+        *reinterpret_cast<f32x4*>(p.adam.P + e) = pp;
+        *reinterpret_cast<f32x4*>(p.adam.M + e) = mm;
+        *reinterpret_cast<f32x4*>(p.adam.V + e) = vv;
+        *reinterpret_cast<u16x4*>(p.adam.Wb + e) = w;
+      }
+    return;
+  }
   constexpr int OB = OUT == OUT_F32 ? 4 : 2;
   typedef typename std::conditional<OB == 4, float, uint16_t>::type out_t;
   typedef out_t out4 __attribute__((ext_vector_type(4), aligned(OB)));
@@ -444,7 +476,7 @@ __global__ __launch_bounds__(64 * WM * WN * KSPL) void gemm_edge_kernel(EdgePara
     }
 }
 
-template <int IN, int OUT, int BM, int BN, int WM, int WN, int KSPL, int PD>
+template <int IN, int OUT, int BM, int BN, int WM, int WN, int KSPL, int PD, bool ADAM = false>
 Status run_edge(const GemmParams& g, hipStream_t s) {
   EdgeParams p{};
   const bool akc = g.a_mode == LD_KCONTIG, bkc = g.b_mode == LD_KCONTIG;
@@ -463,11 +495,12 @@ Status run_edge(const GemmParams& g, hipStream_t s) {
   p.K = (int)g.K;
   p.bias_f32 = g.bias_f32;
   p.act = g.act;
+  p.adam = g.adam;
   p.tiles_m = (p.M + BM - 1) / BM;
   p.tiles_n = (p.N + BN - 1) / BN;
   const unsigned grid = (unsigned)p.tiles_m * (unsigned)p.tiles_n;
   constexpr int threads = 64 * WM * WN * KSPL;
-#define EDGE(A_, B_) gemm_edge_kernel<IN, OUT, BM, BN, WM, WN, KSPL, PD, A_, B_><<<grid, threads, 0, s>>>(p)
+#define EDGE(A_, B_) gemm_edge_kernel<IN, OUT, BM, BN, WM, WN, KSPL, PD, A_, B_, ADAM><<<grid, threads, 0, s>>>(p)
   if (akc && bkc) EDGE(true, true);
   else if (akc) EDGE(true, false);
   else if (bkc) EDGE(false, true);
@@ -512,7 +545,7 @@ Status run_edge_tiles(const GemmParams& g, hipStream_t s) {
 
 bool edge_gemm_ok(const GemmParams& p, int in) {
   const int64_t es = in == IN_F32 ? 4 : 2, ce = 16 / es;
-  if (p.colsum || p.act == ACT_ADAMW || p.c_cs != 1 || !p.apart) return false;
+  if (p.colsum || p.c_cs != 1 || !p.apart) return false;
   if (p.M > INT32_MAX / 2 || p.N > INT32_MAX / 2 || p.K > INT32_MAX / 2 || p.K < ce) return false;
   // 32-bit offsets from a tile's first row, for the up to 256 rows of it
   auto operand_ok = [&](int mode, int64_t ld_k, int64_t ld_mn, int64_t mn) {
@@ -523,8 +556,17 @@ bool edge_gemm_ok(const GemmParams& p, int in) {
   return ((p.M + 63) / 64) * ((p.N + 63) / 64) <= INT32_MAX;
 }
 
+bool edge_splits_k(const GemmParams& p, int in) {
+  const int64_t tiles32 = ((p.M + 31) / 32) * ((p.N + 31) / 32);
+  return tiles32 <= 256 && p.K >= (p.a_mode == LD_KCONTIG ? 2048 : 4096) && edge_gemm_ok(p, in);
+}
+
 Status edge_gemm(GemmParams& p, int in, int out, void* stream) {
   hipStream_t s = as_stream(stream);
+  if (p.act == ACT_ADAMW) {  // edge_splits_k: the configuration of the plain product
+    if (in != IN_BF16 || out != OUT_F32 || p.M % 32 || p.N % 32) return Status::Internal;
+    return run_edge<IN_BF16, OUT_F32, 32, 32, 1, 1, 8, 1, true>(p, s);
+  }
   if (in == IN_F32 && out == OUT_F32) return run_edge_tiles<IN_F32, OUT_F32>(p, s);
   if (in == IN_F16 && out == OUT_F16) return run_edge_tiles<IN_F16, OUT_F16>(p, s);
   if (in == IN_F16 && out == OUT_F32) return run_edge_tiles<IN_F16, OUT_F32>(p, s);

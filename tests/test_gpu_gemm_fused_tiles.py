@@ -78,3 +78,18 @@ def test_ragged_shapes_stay_refused(C, M, N):
     with pytest.raises(RuntimeError, match="InvalidArgument"):
         C.launch_by_id("gemm_adamw_bf16_v0", C.OpKind.GemmAdamW, [a, b, P, m, v, step], [P, m, v, P.bfloat16()], GADW,
                        struct.pack("<iifffff", 0, 0, *HYPER))
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 256, 1984), (256, 256, 2048), (256, 1024, 2048), (512, 512, 4032),
+                                   (512, 512, 4096), (1024, 256, 4096), (512, 768, 4096)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_adamw_of_long_k(C, M, N, K, ta, tb):
+    """Where the plain product splits K the fused one does too: same bits."""
+    test_gemm_adamw_tiles(C, M, N, K, ta, tb)
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 1024, 2048), (256, 1024, 4096), (512, 512, 4096), (768, 512, 2048)])
+@pytest.mark.parametrize("tb", [0, 1])
+def test_dgelu_column_partials_of_long_k(C, M, N, K, tb):
+    """The sums of a product that runs on the K-split tiles."""
+    test_dgelu_column_partials_tiles(C, M, N, K, tb)
