@@ -67,3 +67,19 @@ def test_fused_epilogues_over_a(C):
         runs.append(s + [w])
     for x, y in zip(*runs):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("M,N,K,dt", [(1000, 1000, 1024, "bf16"), (250, 248, 128, "f32"), (2808, 3064, 576, "f16"),
+                                      (129, 127, 64, "bf16"), (517, 700, 519, "f32"), (2561, 2051, 255, "f16")])
+def test_dgelu_over_its_own_pre_activation(C, M, N, K, dt):
+    """At ragged shapes, on tiles moved back or not: each element of Z is read
+    where the output's is stored."""
+    a, b = operands(M, N, K, dt)
+    z = torch.randn((M, N), device="cuda").to(DT[dt])
+    apart = torch.empty_like(z)
+    z64 = z.double().requires_grad_(True)
+    torch.nn.functional.gelu(z64, approximate="tanh").sum().backward()
+    ref = (a.double() @ b.double()) * z64.grad
+    C.op_call(C.OpKind.GemmEpilogue, [a, b, z], [apart], GEPI, struct.pack("<iii", 0, 0, 5))
+    C.op_call(C.OpKind.GemmEpilogue, [a, b, z], [z], GEPI, struct.pack("<iii", 0, 0, 5))
+    assert err(z, ref) < TOL[dt] and err(apart, ref) < TOL[dt]
