@@ -183,12 +183,27 @@ __device__ __forceinline__ void tile_coords_of(int id, int tiles_m, int tiles_n,
   tm = first_m + in_group % gsize;
   tn = in_group / gsize;
 }
+
 // Chunk swizzle of an M/N-contiguous tile in LDS ([k][mn] rows of CPR 16-byte
-// chunks): row k keeps chunk c at c ^ nt_mn_swizzle(k); the reasons are at
-// the tiles' descriptions in gemm.hip.  Rows of 4 chunks (16-bit, 32 wide; the
-// edge kernel's): rows 0-3 and 8-11, read in one 32-lane pass, take different
-// halves of their 64 bytes; fp32 rows of 8 chunks hold one fragment row and
-// stay as they are (rows k and k + 4 share their banks).
+// chunks, ES bytes an element): row k keeps chunk c at c ^ nt_mn_swizzle(k).
+//   16-bit, the 32 lanes of one LDS pass of a transposing fragment read cover 8
+//   K-rows, 0-3 and 8-11 of a fragment's 32 (16 x 16 fragments: MS 16) or 0-7
+//   (32 x 32: groups 0 and 1 at MN + 0 and + 16):
+//     16 chunks or more: with 32 x 32 fragments c ^ 4 (k & 3) keeps the rows on
+//       distinct banks; with 16 x 16 fragments both groups read the same 16 MN
+//       elements 8 rows apart, and the extra 2 ((k >> 3) & 1) term moves the
+//       second group to the other bank half;
+//     8 chunks (64-wide tiles): rows of one parity share a 128-byte bank half,
+//       so the four of them take its four 32-byte slots: chunk pair XOR (bit 1,
+//       bit 3) of k;
+//     4 chunks (32-wide, the edge kernel's): rows 0-3 and 8-11 take different
+//       halves of their 64 bytes.
+//   fp32: a fragment read takes row k and row k + 4 in the two halves of the
+//   wave (32 consecutive floats each).  In rows of 16 chunks or more they sit 8
+//   chunks (32 banks) apart; a row of 8 chunks is one fragment wide and stays as
+//   it is, so the two share their banks.
+// Every 16-bit form keeps rows k and k + 4 (k % 8 < 4) alike, as the fragment's
+// second read (4 rows on) reuses the first one's column.
 template <int MS, int ES = 2, int CPR = 16>
 __device__ __forceinline__ int nt_mn_swizzle(int k) {
   if constexpr (ES == 4) return CPR >= 16 ? 8 * ((k >> 2) & 1) : 0;

@@ -67,9 +67,10 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
 // value).  The empty asm keeps hipcc from fusing an fma and the conversion of
 // its result into v_fma_mixlo/mixhi_f16, which rounds the exact result straight
 // to f16 and can differ from the reference in the last bit.  (A conversion of
-// an operand may be fused: it is exact.)  Every NaN becomes the quiet NaN
-// without payload, with its sign.  Bits of the integer formulation used
-// before, which took ~12 VALU instructions and two branches a value; here 4.
+// an operand may be fused: it is exact.)  In fp32 -> f16 every NaN becomes the
+// quiet NaN without payload, with its sign: the bits of the integer formulation
+// used before, which took ~12 VALU instructions and two branches a value; here
+// 4.  f16 -> fp32 is exact and makes a signalling NaN quiet.
 __device__ __forceinline__ float f16_to_f32(uint16_t h) {
   return static_cast<float>(__builtin_bit_cast(_Float16, h));
 }

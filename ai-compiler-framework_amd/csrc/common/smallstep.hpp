@@ -29,10 +29,17 @@ struct SmallGemm {
   float* bcopy;
 };
 
-// The GEMM dispatcher sends an fp32 problem with fewer than this many
-// 64 x 64 output tiles to small_gemm_f32 (at most 127 such tiles, i.e. 2032
-// tiles of 16 x 16); the lowering's gradient-group jobs use the same bound
-// (SMALL_GEMM_MAX_TILES64 in python/aicf_hip/lower.py).
+// small_gemm_f32 takes fp32 problems with fewer than this many 64 x 64 output
+// tiles (at most 127 such tiles, i.e. 2032 tiles of 16 x 16).  The forward with
+// the copy and the lowering's gradient-group jobs (SMALL_GEMM_MAX_TILES64 in
+// python/aicf_hip/lower.py) use it up to that bound; the GEMM dispatcher sends
+// the larger ones of long K (over 512 tiles of 16 x 16) to the edge kernel's
+// K-split tiles.  The bounds differ on purpose: alone the product is faster
+// there, in a step the launches that the small kernel saves count as much (320 x
+// 784 -> 512 -> 10: 43.0 us in three launches with it, 46.4 in four with the
+// forward on the other, 900 x 500 -> 400 -> 10 52.3 and 53.4, 512 x 512 -> 512
+// -> 10 43.6 and 41.9).  Such a forward has the other kernel's values to fp32
+// rounding, not to the bit.
 constexpr int64_t kSmallGemmMaxTiles64 = 128;
 
 // True when small_gemm_f32 takes the problem (sizes within int range, unit

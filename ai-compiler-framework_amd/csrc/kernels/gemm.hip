@@ -755,24 +755,12 @@ struct NTSched {
 //     c ^ nt_mn_swizzle(k).  A fragment (MS MN x 16 or 32 K) is two
 //     ds_read_b64_tr_b16 per 16-lane group: lane j points at row k0 + j/4,
 //     elements m + 4 (j%4) .. +3, and the transposing read hands lane i the
-//     four K values of element m + i.  The 32 lanes of one LDS pass read 8
-//     K-rows: with 32 x 32 fragments (groups 0 and 1 at MN + 0 and + 16)
-//     c ^ 4 (k & 3) keeps them on distinct banks; with 16 x 16 fragments
-//     both groups read the same 16 MN elements 8 rows apart, and the extra
-//     2 ((k >> 3) & 1) term moves the second group to the other bank half.
+//     four K values of element m + i.
 //   K-contiguous rows are 128 B: the chunk c ^ ((r >> 1) & 7) keeps the 32
 //     (or 16) rows of one fragment read on all 64 banks.
 // Loads are buffer loads straight into LDS with per-lane offsets fixed for
 // the whole K loop (the K advance is the scalar offset); the host checks that
 // the bytes a resource spans fit a signed 32-bit offset.
-// fp32 (ES 4): a fragment read takes one row k and the row k + 4 in the two
-// halves of the wave (32 consecutive floats each), so rows k and k + 4 sit
-// 8 chunks (32 banks) apart.  16-bit rows of 8 chunks (64-wide tiles): a
-// transposing read's 32-lane pass covers rows {0-3, 8-11} (+ 16 k) with 32
-// bytes each; rows of one parity share a 128-byte bank half, so the four of
-// them take the four 32-byte slots: chunk pair XOR (bit 1, bit 3) of k.
-// Every form keeps rows k and k + 4 (k % 8 < 4) alike, as the fragment's
-// second read (4 rows on) reuses the first one's column.
 template <bool KC, int BMN, int NW, int ES>
 struct NTOperand {
   static constexpr int BYTES = BMN * 128;            // a stage holds 128 B of K per row
@@ -1359,8 +1347,9 @@ Status run_nt(const GemmParams& g, hipStream_t s) {
 // epilogue (none, ReLU, GELU): four waves of 128 x 128, one per SIMD, which
 // issue the MFMAs back to back.  Everything else: eight waves of 128 x 64; the
 // GELU (two outputs) and dGELU (pre-activation read) epilogues move twice
-// the bytes per wave with four waves, and f16's integer-rounded epilogue
-// needs the registers.
+// the bytes per wave with four waves.  f16 keeps eight: four take 4% less on
+// several rounds of long K (8192^3 770 us, 740) but 6-9% more at K <= 1024
+// (8192 x 4096 x 1024 61.2, 65.1, with GELU 69.6, 75.0).
 template <int IN, int OUT>
 Status run_nt256(const GemmParams& g, hipStream_t s) {
   if constexpr (IN == IN_BF16) {

@@ -511,12 +511,12 @@ __device__ __forceinline__ void ln_bwd_columns(const LnBwd<T>& a, int block, flo
   }
 }
 
-// f16 [1500, 1000]: 8.0 us against 146 for a dx kernel and a column kernel of
-// N / 64 workgroups that walk all rows.
 // Backward in one launch: the first `row_blocks` workgroups compute dx, a row
 // per LPR lanes; the others dgamma and dbeta, reading x and dy a second time,
 // which comes from the caches for the sizes this kernel is used at.  reserved
-// (see LnBwd): dx of the last RS rows of each chunk instead of all rows.
+// (see LnBwd): dx of the last RS rows of each chunk instead of all rows.  f16
+// [1500, 1000]: 8.0 us against 146 for a dx kernel and a column kernel of N / 64
+// workgroups that walk all rows.
 template <typename T, int LPR, int VPT>
 __global__ __launch_bounds__(ln_threads(LPR)) void ln_bwd_kernel(LnBwd<T> a, int row_blocks, bool reserved) {
   constexpr int RPB = ln_threads(LPR) / LPR;
@@ -544,13 +544,12 @@ __global__ __launch_bounds__(kLnColThreads) void ln_bwd_columns_kernel(LnBwd<T> 
   ln_bwd_columns<T>(a, blockIdx.x, red);
 }
 
-// f32 [8192, 4096]: 66 us (6.1 TB/s of x, dy and dx), 78 with the finish and
-// the reserved rows, against 1040 for the two separate kernels; bound by HBM.
 // Fused backward: workgroup w owns the rows of chunk w, G = 1024 / LPR groups
 // of lanes taking every G-th of them, and a lane keeps the dgamma and dbeta
 // sums of its columns in registers over all its rows.  The groups' sums are
 // added in LDS by a fixed-order tree and written to the chunk's reserved rows
-// of dx.
+// of dx.  f32 [8192, 4096]: 66 us (6.1 TB/s of x, dy and dx), 78 with the finish
+// and the reserved rows, against 1040 for the two separate kernels; bound by HBM.
 template <typename T, int LPR, int VPT>
 __global__ __launch_bounds__(1024) void ln_bwd_fused_kernel(LnBwd<T> a) {
   constexpr int V = kVec<T>, G = 1024 / LPR, COLS = LPR * VPT * V;
@@ -820,8 +819,11 @@ Status ln_bwd_run(LnBwd<T> a, LnOut where, hipStream_t s) {
   // 256 MB MALL) the second read of the one-launch form comes from the caches
   // and its two launches less count more, until its N / 2 V column workgroups
   // have too many rows each: f32 [2048, 632] 10.6 us against 13.9 fused,
-  // [4096, 512] 22.7 against 13.1, [16384, 100] 50 against 18.  Fewer than 8
-  // rows a chunk would leave a quarter or more of the rows to the last launch.
+  // [4096, 512] 22.7 against 13.1, [16384, 100] 50 against 18.  8 rows a chunk at
+  // least: the last launch reads the RS reserved ones of each again, at 8 rows a
+  // quarter of x and dy in fp32 and half or more in f16, where the fused form is
+  // the faster one all the same (f16 [2048, 8192] 45 us against 68, [2049, 8200]
+  // 61 against 67, [2560, 4096] 30 against 42).
   constexpr int64_t kFusedBytes = 16 << 20;
   constexpr int kChunks = 256, kFusedRows = 3584;
   if (where == LnOut::Apart && nv <= 2048 && M >= 8 * kChunks && ((int64_t)M * N * (int64_t)sizeof(T) >= kFusedBytes || M >= kFusedRows)) {
@@ -1113,12 +1115,13 @@ __global__ __launch_bounds__(T) void bn_bwd_reg_kernel(const uint16_t* x, const 
   }
 }
 
-// [32, 64, 56, 56]: 5.2 + 2.8 + 7.0 us forward and 6.2 + 1.8 + 8.2 backward,
-// against 342 and 366 with one workgroup a channel (64 of 256 CUs), 2-byte
-// loads and a 64-bit division an element; launches are now half of it.
 // Large channels: chunk p of channel c is kBNChunk vectors, one workgroup
 // (p, c) each, whose two partial values go to part[c P + p]: forward, the
 // chunk's mean and centred square sum; backward, its sums of dy and dy xhat.
+// [32, 64, 56, 56]: 5.2 + 2.8 + 7.0 us in the three kernels forward and 6.2 +
+// 1.8 + 8.2 backward, against 342 and 366 with one workgroup a channel (64 of
+// 256 CUs), 2-byte loads and a 64-bit division an element; launches are now half
+// of it.
 constexpr int kBNVpt = 4, kBNChunk = 256 * kBNVpt;
 
 template <int V>

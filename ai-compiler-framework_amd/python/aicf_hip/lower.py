@@ -439,7 +439,7 @@ def _numel_shape(shape) -> int:
 
 
 def gemm_adamw_eligible(M: int, N: int, K: int) -> bool:
-    """Shapes the fused kernel (256 x 256 tiles) covers."""
+    """Shapes the fused epilogue covers."""
     return M % 256 == 0 and N % 256 == 0 and K % 64 == 0 and M > 0 and N > 0 and K > 0
 
 
@@ -455,7 +455,7 @@ def fuse_optimizer_into_gemms(ir: IRGraph, lowered: Lowered) -> Lowered:
     (the fused kernels read the incremented counter, as the flat step does).
     The updates are bit-identical to the unfused plan: the epilogue applies
     the same AdamW expression to the same fp32 accumulators the GEMM would
-    have stored."""
+    have stored (the dispatcher splits K for both alike)."""
     kind = lambda it: str(it.get("op", "")).strip().lower()  # noqa: E731
     ad = [i for i, it in enumerate(lowered) if kind(it) == "adamw_step"]
     if len(ad) != 1 or len(lowered[ad[0]]["outputs"]) != 4:
@@ -538,11 +538,11 @@ def fuse_optimizer_into_gemms(ir: IRGraph, lowered: Lowered) -> Lowered:
 def fuse_colsum_into_dgelu(ir: IRGraph, lowered: Lowered) -> Lowered:
     """StageC' (not in the reference): reduce_sum(dz) -> (db, workspace) over
     the output of a bf16 dGELU gemm_epilogue becomes part of that GEMM (GEPI
-    kind 6: outputs dz, db, workspace).  Only where the GEMM runs on the
-    256 x 256 tiles that carry the column sums (bf16 2-D operands, M and N
-    multiples of 256, K of 64) and the reduce_sum has a [P >= M/256, N] fp32
-    workspace; db then sums one partial per 256-row tile instead of the
-    two-pass column sum's order (equal to fp32 rounding)."""
+    kind 6: outputs dz, db, workspace).  Only where the GEMM carries the
+    column sums (bf16 2-D operands, M and N multiples of 256, K of 64) and the
+    reduce_sum has a [P >= M/256, N] fp32 workspace; db then sums one partial
+    per 256 rows instead of the two-pass column sum's order (equal to fp32
+    rounding)."""
     kind = lambda it: str(it.get("op", "")).strip().lower()  # noqa: E731
     producer = {}
     for i, it in enumerate(lowered):
@@ -713,9 +713,10 @@ def fuse_step_tail(ir: IRGraph, lowered: Lowered) -> Lowered:
 # ---------------------------------------------------------------- StageF
 GJ_GEMM, GJ_COLSUM, GJ_MEAN, GJ_STEP = 0, 1, 2, 3
 MAX_GROUP_JOBS = 8
-# fp32 GEMMs with fewer 64 x 64 output tiles than this run on the small-GEMM
-# kernel (kSmallGemmMaxTiles64 in csrc/common/smallstep.hpp, which the GEMM
-# dispatcher uses); only those are grouped as gradient-group jobs
+# fp32 GEMMs with fewer 64 x 64 output tiles than this can run on the
+# small-GEMM kernel (kSmallGemmMaxTiles64 in csrc/common/smallstep.hpp, where the
+# reasons are); only those are grouped as gradient-group jobs.  The dispatcher
+# sends the larger of them elsewhere when they run alone
 SMALL_GEMM_MAX_TILES64 = 128
 MAX_ADAMW_TENSORS = 8
 
