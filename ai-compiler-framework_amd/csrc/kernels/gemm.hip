@@ -1401,12 +1401,16 @@ bool nt_eligible(const GemmParams& p, int BM, int BN, bool mn_ok) {
       // here); 16-bit from K = 1024 on, or 768 with one output and a 128 x 128
       // tile a CU (bf16 2048 x 2880 x 1024 30.1 us on 64 x 64, 16.0 here, x 768
       // 17.0, 12.9, but 1600 x 1600 x 768 8.7, 9.7), and 256 x 256 only while
-      // they take one round of the CUs (2944 x 2944 x 1024 28.2 on 128 x 128,
-      // 24.7; 4224 x 4224 x 1024 41.5, 43.1)
+      // they take one round of the CUs (2944 x 2944 x 1024 NN 28.6 on 128 x 128,
+      // 24.7; 4224 x 4224 x 1024 47.2, 49.4) and, beside 128 x 128 ones, with two
+      // outputs or a pre-activation from K = 1536 on (8192 x 1152 x 1024 NT with
+      // both GELU outputs 30.3, 32.1)
       const int64_t tiles128 = ((p.M + 127) / 128) * ((p.N + 127) / 128);
       const bool one_out = p.act == ACT_NONE || p.act == ACT_RELU || (p.act == ACT_GELU && !p.aux);
       if (IN == IN_F32 || p.K < (one_out && tiles128 >= 256 ? 768 : 1024)) return false;
-      if (BM == 256 && ((p.M + 255) / 256) * ((p.N + 255) / 256) > 256) return false;
+      if (BM == 256 && (((p.M + 255) / 256) * ((p.N + 255) / 256) > 256 ||
+                        (!one_out && p.M % 128 == 0 && p.N % 128 == 0 && p.K < 1536)))
+        return false;
     }
     const int64_t rows = (p.M + BM - 1) / BM * BM, cols = (p.N + BN - 1) / BN * BN;
     if ((double)rows * cols > 1.25 * (double)p.M * p.N) return false;
