@@ -1367,7 +1367,9 @@ bool bn_outputs_apart(const TensorDesc* in, int ni, const TensorDesc* out, int n
     else if (total <= 512 * 8) { CALL(V, 512, 8); }     \
     else { CALL(V, 1024, 8); }                          \
   }
-constexpr int64_t kBNRegVecs = 1024 * 8;
+// The runtime counts a grid's lanes in 32 bits and starts too few workgroups,
+// without an error, above that: no more channels of over 256 lanes than fit.
+bool bn_in_registers(int64_t total, int64_t C) { return total <= 1024 || (total <= 1024 * 8 && C < 1 << 22); }
 
 template <int V>
 dim3 bn_apply_grid(const BNShape& sh) {
@@ -1379,7 +1381,7 @@ Status bn_fwd_train(const uint16_t* x, const uint16_t* g, const uint16_t* b, uin
                     BNShape sh, float eps, bool apart, hipStream_t s) {
   sh.HV = sh.HW / V;
   const int64_t total = (int64_t)sh.N * sh.HV;
-  if (total <= kBNRegVecs) {
+  if (bn_in_registers(total, sh.C)) {
 #define BN_FWD(VV, T, VPT) bn_fwd_reg_kernel<VV, T, VPT><<<(unsigned)sh.C, T, 0, s>>>(x, g, b, y, sm, sr, sh, eps)
     BN_REG_BY_SIZE(V, total, BN_FWD)
 #undef BN_FWD
@@ -1414,7 +1416,7 @@ Status bn_bwd_run(const uint16_t* x, const uint16_t* dy, const uint16_t* g, cons
                   uint16_t* dx, float* dg, float* db, BNShape sh, bool apart, hipStream_t s) {
   sh.HV = sh.HW / V;
   const int64_t total = (int64_t)sh.N * sh.HV;
-  if (total <= kBNRegVecs) {
+  if (bn_in_registers(total, sh.C)) {
 #define BN_BWD(VV, T, VPT) \
   bn_bwd_reg_kernel<VV, T, VPT><<<(unsigned)sh.C, T, 0, s>>>(x, dy, g, sm, sr, dx, dg, db, sh)
     BN_REG_BY_SIZE(V, total, BN_BWD)

@@ -11,7 +11,7 @@ import pytest
 import torch
 
 import oracle as orc
-from test_gpu_norm import LNEP, dev, host, rng
+from test_gpu_norm import BNEP, LNEP, dev, host, rng
 
 pytestmark = pytest.mark.gpu
 
@@ -101,3 +101,24 @@ def test_rows_of_more_than_a_grid(C, n, times, cols):
     assert orc.rel_err(host(rl[:n]), row) < 1e-5 and same(rl, n)
     assert orc.rel_err(host(y[:n]), d / R) < 1e-5 and same(y, n)
     assert abs(float(loss) - row.mean()) < 1e-5 * abs(row.mean())
+
+
+def test_batchnorm_of_more_channels_than_a_grid(C):
+    """2^22 channels at 1024 lanes each, in place; all have the values -1 and
+    +1 in turn, so that mean and variance are known."""
+    n, Cc = 4099, (1 << 22) + 1
+    if torch.cuda.mem_get_info()[0] < 60 << 30:
+        pytest.skip("34 GB of channels")
+    x = torch.empty((1, Cc, 1, n), device="cuda", dtype=torch.float16)
+    x.view(Cc, n)[:, ::2] = -1
+    x.view(Cc, n)[:, 1::2] = 1
+    mu = -1 / n
+    r = (1 - mu * mu + 1e-5) ** -0.5
+    mean, rstd = torch.zeros(Cc, device="cuda"), torch.zeros(Cc, device="cuda")
+    C.op_call(C.OpKind.BatchNormFwd, [x], [x, mean, rstd], BNEP, struct.pack("<fI", 1e-5, 0))
+    assert float((mean - mu).abs().max()) < 1e-5 and float((rstd / r - 1).abs().max()) < 1e-5
+    want = torch.full((n,), (1 - mu) * r, device="cuda")
+    want[::2] = (-1 - mu) * r
+    assert all(float((c.float() - want).abs().max()) < 2e-3 for c in x.view(Cc, n).split(1 << 18))
+    del x
+    torch.cuda.empty_cache()
