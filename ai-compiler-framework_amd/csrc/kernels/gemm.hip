@@ -1399,15 +1399,17 @@ bool nt_eligible(const GemmParams& p, int BM, int BN, bool mn_ok) {
       // exact smaller tiles exist: fp32 is bound by its MFMAs and loses by
       // every row computed twice (4160 x 4160 x 512 NN 141 us on 64 x 64, 242
       // here); 16-bit from K = 1024 on, or 768 with one output and a 128 x 128
-      // tile a CU (bf16 2048 x 2880 x 1024 30.1 us on 64 x 64, 16.0 here, x 768
-      // 17.0, 12.9, but 1600 x 1600 x 768 8.7, 9.7), and 256 x 256 only while
-      // they take one round of the CUs (2944 x 2944 x 1024 NN 28.6 on 128 x 128,
-      // 24.7; 4224 x 4224 x 1024 47.2, 49.4) and, beside 128 x 128 ones, with two
-      // outputs or a pre-activation from K = 1536 on (8192 x 1152 x 1024 NT with
-      // both GELU outputs 30.3, 32.1)
+      // tile a CU (bf16 2048 x 2880 x 1024 NN 29.7 us on 64 x 64, 15.6 here, x 768
+      // 17.0, 12.9, but 1600 x 1600 x 768 7.6, 8.4), or 512 with eight of them
+      // (5824 x 5824 x 512 76, 46; 6464 x 3136 x 512 with both GELU outputs loses
+      // 20%); and 256 x 256 only while they take one round of the CUs (2944 x 2944
+      // x 1024 NN 28.6 on 128 x 128, 24.7; 4224 x 4224 x 1024 47.2, 49.4) and,
+      // beside 128 x 128 ones, with two outputs or a pre-activation from K = 1536
+      // on (8192 x 1152 x 1024 NT with both GELU outputs 30.3, 32.1)
       const int64_t tiles128 = ((p.M + 127) / 128) * ((p.N + 127) / 128);
       const bool one_out = p.act == ACT_NONE || p.act == ACT_RELU || (p.act == ACT_GELU && !p.aux);
-      if (IN == IN_F32 || p.K < (one_out && tiles128 >= 256 ? 768 : 1024)) return false;
+      const int64_t from = tiles128 >= 2048 ? 512 : one_out && tiles128 >= 256 ? 768 : 1024;
+      if (IN == IN_F32 || p.K < from) return false;
       if (BM == 256 && (((p.M + 255) / 256) * ((p.N + 255) / 256) > 256 ||
                         (!one_out && p.M % 128 == 0 && p.N % 128 == 0 && p.K < 1536)))
         return false;

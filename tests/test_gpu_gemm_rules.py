@@ -47,6 +47,12 @@ def test_shapes_of_whole_smaller_tiles(C, M, N, K, dt):
     check(C, M, N, K, dt, (3, 5) if dt != "bf16_f32" else ())
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("K", [448, 512])
+def test_many_tiles_of_whole_64s(C, K, dt):
+    check(C, 5824, 5696, K, dt)
+
+
 @pytest.mark.parametrize("M,N,K", [(2048, 1536, 1024), (2048, 1792, 512), (2048, 1792, 544), (2048, 2048, 512),
                                    (2048, 2048, 1056), (2048, 2176, 1024), (3072, 2048, 128)])
 def test_fp32_tiles_by_the_fullest_cu(C, M, N, K):
